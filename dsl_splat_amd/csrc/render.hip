@@ -33,6 +33,8 @@
 // most 64 - 8 channels, so its gradient entries fit the 64 lanes of one
 // wavefront sum, and channels beyond it enter the dot product from global
 // memory.  Further windows add only their channels' feature gradients.
+#include <type_traits>
+
 #include "common.hpp"
 
 #ifndef GS3D_FWD_PIX
@@ -81,19 +83,25 @@ struct PixFor {
                                             : 1;
 };
 
-// Tile-local coordinates of pixel k of thread t.
+// The wavefronts of a tile each own a rectangle of its pixels, 16 x 8 at two
+// pixels per lane and 8 x 8 at one.  A Gaussian touches a square of 8 x 8
+// pixels less often than a strip of 16 x 4: a 256x256 frame's backward took
+// 138 against 142 us, a 637x421 frame's with 9 channels 217 against 238.
+template <int PIX>
+struct TileWaves {
+    static constexpr int count = kTilePixels / PIX / 64;
+    static constexpr int cols = PIX == 1 ? 8 : 16;
+    static constexpr int rows = 64 * PIX / cols;
+    static constexpr int across = kTile / cols;
+};
+
+// Tile-local coordinates of pixel k of thread t: a lane owns PIX neighbours
+// of a row, 8 lanes a row of the wavefront's rectangle.
 template <int PIX>
 GS3D_DEV void pixel_of(int t, int k, int& x, int& y) {
-    if (PIX == 1) {
-        x = t & 15;
-        y = t >> 4;
-    } else if (PIX == 2) {
-        x = 2 * (t & 7) + k;
-        y = t >> 3;
-    } else {
-        x = 2 * (t & 7) + (k & 1);
-        y = 2 * (t >> 3) + (k >> 1);
-    }
+    const int w = t >> 6, lane = t & 63;
+    x = (w % TileWaves<PIX>::across) * TileWaves<PIX>::cols + PIX * (lane & 7) + k;
+    y = (w / TileWaves<PIX>::across) * TileWaves<PIX>::rows + (lane >> 3);
 }
 
 struct TileInfo {
@@ -133,19 +141,79 @@ GS3D_DEV TileInfo tile_info(const gs3d_render_args& a, int tile) {
 
 GS3D_DEV TileInfo tile_info(const gs3d_render_args& a) { return tile_info(a, tile_of_block(blockIdx.x, gridDim.x)); }
 
-// Lowest power at which opacity o can still give alpha >= 1/255 (see the
-// file comment); +inf rejects everything (o <= 0), -inf rejects nothing.
-GS3D_DEV float power_cutoff(float o) {
-    if (o > 0.0f) return -__logf(255.0f * o) - 0.01f;
-    return o <= 0.0f ? __builtin_inff() : -__builtin_inff();
+// The blends work with the negated exponent, -power: alpha = o e^power can
+// only reach 1/255 where -power <= ln(255 o) + 0.01 (see the file comment).
+// -inf rejects everything (o <= 0).  Beyond 86 the exponential is zero, so a
+// finite opacity rejects there in any case; a NaN or infinite one accepts
+// every pixel with -power >= 0 (min(0.99, NaN) = 0.99), and +inf says so.
+GS3D_DEV float exponent_limit(float o) {
+    if (o > 0.0f) return o < __builtin_inff() ? sel_min(__logf(255.0f * o) + 0.01f, 86.0f) : __builtin_inff();
+    return o <= 0.0f ? -__builtin_inff() : __builtin_inff();
 }
 
-// The wavefronts of a tile each own a horizontal strip of its rows.
-template <int PIX>
-struct TileWaves {
-    static constexpr int count = kTilePixels / PIX / 64;
-    static constexpr int rows = kTile / count;
-};
+// -power of the blend, from the two products of dy: the negation of
+// blend_power bit for bit (rounding is symmetric in the sign), except that a
+// zero is always +0: accepts() compares bit patterns.
+GS3D_DEV float blend_exponent(float a, float b, float dx, float dy, float c_dy_dy) {
+    const float q = __builtin_fmaf(a * dx, dx, c_dy_dy);
+    return __builtin_fmaf(0.5f, q, __builtin_fmaf(b * dx, dy, 0.0f));
+}
+
+// 0 <= x <= limit for a positive limit, in one compare: positive floats order
+// as their bit patterns, negative numbers and NaNs lie above all of them.
+GS3D_DEV bool accepts(float x, float limit) { return __float_as_uint(x) <= __float_as_uint(limit); }
+
+// blend_exp(-x) for 0 <= x <= 86 without its range check: the same reduction
+// and polynomial.  The integer k comes from adding 1.5 * 2^23 (the sum rounds
+// t to the nearest integer, ties to even, as rint does) and stays in the low
+// bits of that sum, whose shift into the exponent field is the exact scaling
+// (every result is a normal number).  rndne, cvt and ldexp run at half the
+// rate of an add on this part, and the check is a compare and a select more.
+GS3D_DEV float blend_exp_neg(float x) {
+    const float z = x * -1.44269502e+00f + 12582912.0f;
+    const float k = z - 12582912.0f;
+    float r = __builtin_fmaf(k, -6.93145752e-01f, -x);
+    r = __builtin_fmaf(k, -1.42860677e-06f, r);
+    float p = 1.98412701e-04f;
+    p = __builtin_fmaf(p, r, 1.38888892e-03f);
+    p = __builtin_fmaf(p, r, 8.33333377e-03f);
+    p = __builtin_fmaf(p, r, 4.16666679e-02f);
+    p = __builtin_fmaf(p, r, 1.66666672e-01f);
+    p = __builtin_fmaf(p, r, 5.00000000e-01f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    return __uint_as_float(__float_as_uint(p) + (__float_as_uint(z) << 23));
+}
+
+// An exponent beyond 86, accepted only because the opacity is not finite,
+// kept in blend_exp_neg's range (alpha is 0.99 whatever the exponential is).
+// Opaque, so that the rare case stays a branch instead of selects for
+// everyone.
+GS3D_DEV float clamp_exponent(float x) {
+    asm volatile("v_min_f32 %0, 0x42ac0000, %0" : "+v"(x));
+    return x;
+}
+
+// Lane masks of the whole wavefront as scalars, and a select by one.  Written
+// out as the three-operand form: consecutive two-operand selects on vcc issue
+// six times slower than others on this part (23 against 4.5 cycles in a loop
+// of them).
+GS3D_DEV uint64_t lanes(bool v) { return __builtin_amdgcn_ballot_w64(v); }
+GS3D_DEV float select(uint64_t mask, float yes, float no) {
+    float r;
+    asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(no), "v"(yes), "s"(mask));
+    return r;
+}
+GS3D_DEV float select0(uint64_t mask, float yes) {
+    float r;
+    asm("v_cndmask_b32_e64 %0, 0, %1, %2" : "=v"(r) : "v"(yes), "s"(mask));
+    return r;
+}
+GS3D_DEV int select(uint64_t mask, int yes, int no) {
+    int r;
+    asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(no), "v"(yes), "s"(mask));
+    return r;
+}
 
 // Minimum over dx in [lo, hi] of Q = a dx^2 + 2 b dx dy + c dy^2 at a fixed
 // dy (a > 0): Q at the clamped stationary point -b dy / a.  The reciprocal
@@ -156,10 +224,10 @@ GS3D_DEV float edge_min(float a, float inv_a, float b, float c, float dy, float 
     return (a * d + 2.0f * b * dy) * d + c * dy * dy;
 }
 
-// Bit w is set unless every pixel of wavefront w's strip is certain to reject
-// the Gaussian: the ellipse {power >= cut}, its quadratic form Q widened by
-// 1% + 0.01, misses the strip's rectangle of pixel centres -- first by its
-// bounding box (widened by 0.01 px), then exactly: the strip is kept when
+// Bit w is set unless every pixel of wavefront w's rectangle is certain to
+// reject the Gaussian: the ellipse {-power <= limit}, its quadratic form Q
+// widened by 1% + 0.01, misses the rectangle of pixel centres -- first by its
+// bounding box (widened by 0.01 px), then exactly: the rectangle is kept when
 // the centre lies inside the rectangle or Q's minimum over one of the
 // rectangle's four edges is within the widened bound.  Float32 evaluation of
 // Q is off by at most about 8 * 2^-24 * (a + c) |d|^2, below 2e-4 Q for the
@@ -173,11 +241,11 @@ GS3D_DEV float edge_min(float a, float inv_a, float b, float c, float dy, float 
 // ones, overflowing products and NaNs are never culled.  Rejected pairs change
 // no output, so culling leaves every result identical.
 template <int PIX>
-GS3D_DEV uint32_t strip_mask(float2 xy, float4 con, float cut, int x0, int y0) {
-    constexpr int NW = TileWaves<PIX>::count, ROWS = TileWaves<PIX>::rows;
-    constexpr uint32_t all = (1u << NW) - 1u;
-    const float q = -2.0f * cut;  // power >= cut  <=>  a dx^2 + 2 b dx dy + c dy^2 <= q
-    if (!(q > 0.0f) && q == q) return 0u;  // nothing passes the cutoff
+GS3D_DEV uint32_t strip_mask(float2 xy, float4 con, float limit, int x0, int y0) {
+    using W = TileWaves<PIX>;
+    constexpr uint32_t all = (1u << W::count) - 1u;
+    const float q = 2.0f * limit;  // -power <= limit  <=>  a dx^2 + 2 b dx dy + c dy^2 <= q
+    if (!(q > 0.0f) && q == q) return 0u;  // nothing passes the limit
     const float a = con.x, b = con.y, c = con.z;
     const float ac = a * c;
     const float det = ac - b * b;
@@ -187,17 +255,17 @@ GS3D_DEV uint32_t strip_mask(float2 xy, float4 con, float cut, int x0, int y0) {
     const float s = (q * 1.01f + 0.01f) * __builtin_amdgcn_rcpf(det);
     const float hx = __builtin_amdgcn_sqrtf(s * c) + 0.01f;
     const float hy = __builtin_amdgcn_sqrtf(s * a) + 0.01f;
-    if (xy.x + hx < (float)x0 || xy.x - hx > (float)(x0 + kTile - 1)) return 0u;
     const float bound = q * 1.01f + 0.01f;
     const float inv_a = __builtin_amdgcn_rcpf(a), inv_c = __builtin_amdgcn_rcpf(c);
-    // Centre minus pixel over the tile's columns.
-    const float dx_lo = xy.x - (float)(x0 + kTile - 1), dx_hi = xy.x - (float)x0;
     uint32_t m = 0u;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-        const float lo = (float)(y0 + w * ROWS), hi = (float)(y0 + w * ROWS + ROWS - 1);
-        if (xy.y + hy < lo || xy.y - hy > hi) continue;
-        const float dy_lo = xy.y - hi, dy_hi = xy.y - lo;
+    for (int w = 0; w < W::count; ++w) {
+        const float x_lo = (float)(x0 + (w % W::across) * W::cols), x_hi = x_lo + (float)(W::cols - 1);
+        const float y_lo = (float)(y0 + (w / W::across) * W::rows), y_hi = y_lo + (float)(W::rows - 1);
+        if (xy.x + hx < x_lo || xy.x - hx > x_hi || xy.y + hy < y_lo || xy.y - hy > y_hi) continue;
+        // Centre minus pixel over the rectangle.
+        const float dx_lo = xy.x - x_hi, dx_hi = xy.x - x_lo;
+        const float dy_lo = xy.y - y_hi, dy_hi = xy.y - y_lo;
         bool keep = dx_lo <= 0.0f && dx_hi >= 0.0f && dy_lo <= 0.0f && dy_hi >= 0.0f;  // centre inside
         if (!keep) {
             const float e0 = edge_min(a, inv_a, b, c, dy_lo, dx_lo, dx_hi);
@@ -220,15 +288,20 @@ template <int CH>
 struct alignas(16) StagedRec {
     float4 con;
     float2 xy;
-    float cut;
-    float pad;
+    float limit;  // exponent_limit
+    int entry;    // list position, 1-based
     float f[CH];
 };
+
+// Strip-mask bit of a Gaussian whose opacity (kStrange) is not finite or one
+// of whose staged channels (kStrangeColor) is not: the blend loops take their
+// cases apart.
+constexpr uint32_t kStrange = 1u << 31, kStrangeColor = 1u << 30;
 
 // Stage one Gaussian's centre, conic, cutoff, strip mask and the channels
 // [c0, c0 + CH) of its channel vector (zero beyond D').
 template <int CH, int PIX, bool LAUNDER = false>
-GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32_t g, int slot, int c0,
+GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32_t g, int slot, int entry, int c0,
                              StagedRec<CH>* s_g, uint32_t* s_mask) {
     const int view = t.view;
     const int64_t row = (int64_t)view * a.n + g;
@@ -256,8 +329,9 @@ GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32
     StagedRec<CH>& rec = s_g[slot];
     rec.con = con;
     rec.xy = xy;
-    const float cut = power_cutoff(con.w);
-    rec.cut = cut;
+    const float limit = exponent_limit(con.w);
+    rec.limit = limit;
+    rec.entry = entry;
     int x0 = t.x0, y0 = t.y0;
     if constexpr (LAUNDER) {
         // The tile origin passes through an opaque scalar move, so that the
@@ -266,9 +340,18 @@ GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32
         // into VGPRs that stay live over the whole traversal.
         asm volatile("" : "+s"(x0), "+s"(y0));
     }
-    s_mask[slot] = strip_mask<PIX>(xy, con, cut, x0, y0);
+    uint32_t mask = strip_mask<PIX>(xy, con, limit, x0, y0);
+    // The channels' magnitudes, largest first: a NaN survives the integer
+    // maximum of the bit patterns.
+    uint32_t top = 0u;
 #pragma unroll
-    for (int c = 0; c < CH; ++c) rec.f[c] = v[c];
+    for (int c = 0; c < CH; ++c) {
+        rec.f[c] = v[c];
+        top = max(top, __float_as_uint(v[c]) & 0x7FFFFFFFu);
+    }
+    if (top >= 0x7F800000u) mask |= kStrangeColor;
+    if (limit == __builtin_inff()) mask |= kStrange;
+    s_mask[slot] = mask;
 }
 
 // 0.0f that the compiler cannot see through (a register written by an
@@ -294,7 +377,8 @@ template <int CH>
 struct Staged {
     float2 xy;
     float4 con;
-    float cut;
+    float limit;
+    int entry;
     float f[CH];
 };
 
@@ -304,7 +388,8 @@ GS3D_DEV Staged<CH> load_staged(int j, const StagedRec<CH>* s_g) {
     Staged<CH> g;
     g.xy = rec.xy;
     g.con = rec.con;
-    g.cut = rec.cut;
+    g.limit = rec.limit;
+    g.entry = rec.entry;
 #pragma unroll
     for (int c = 0; c < CH; ++c) g.f[c] = rec.f[c];
     return g;
@@ -367,13 +452,13 @@ GS3D_DEV void flush_statistics(const gs3d_render_stats_args& st, int view, int n
 // from st.sum_mask.
 template <int PIX, int RB, int KINDS>
 GS3D_DEV void observe_statistics(const gs3d_render_stats_args& st, int dst_r, float* slot,
-                                 const bool (&acc)[PIX], const float (&w)[PIX], const float (&val)[PIX][RB],
+                                 const uint64_t (&acc)[PIX], const float (&w)[PIX], const float (&val)[PIX][RB],
                                  bool finite, int lane) {
     float e[RB];
     if (finite) {
         float one[PIX];
 #pragma unroll
-        for (int k = 0; k < PIX; ++k) one[k] = acc[k] ? 1.0f : 0.0f;
+        for (int k = 0; k < PIX; ++k) one[k] = select0(acc[k], 1.0f);
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
             // wave-uniform; a compile-time constant for KINDS >= 0
@@ -390,7 +475,7 @@ GS3D_DEV void observe_statistics(const gs3d_render_stats_args& st, int dst_r, fl
             float v = 0.0f;
 #pragma unroll
             for (int k = 0; k < PIX; ++k) {
-                const bool hit = acc[k] && val[k][r] != 0.0f;
+                const bool hit = ((acc[k] >> lane) & 1) && val[k][r] != 0.0f;
                 v += hit ? (is_sum ? val[k][r] * w[k] : 1.0f) : 0.0f;
             }
             e[r] = v;
@@ -433,12 +518,13 @@ GS3D_DEV void observe_statistics(const gs3d_render_stats_args& st, int dst_r, fl
 // capped launch.  Only the instantiations that use them carry the stop
 // tracking and the loop.
 template <int CH, int PIX, int MODE, int RB = 1, int KINDS = -1, int LISTS = 0>
-__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 6 : CH <= 8 ? 5 : 1))) void render_fwd_kernel(gs3d_render_args a, gs3d_render_stats_args st, int c0, unsigned long long* counts) {
+__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 6 : CH <= 8 ? 5 : CH <= 36 ? 3 : 1))) void render_fwd_kernel(gs3d_render_args a, gs3d_render_stats_args st, int c0, unsigned long long* counts) {
     constexpr bool STATS = MODE == 1, COUNTS = MODE == 2;
     constexpr int NT = kTilePixels / PIX;
     constexpr int B = Batch<CH>::size;
     __shared__ StagedRec<CH> s_g[B];
     __shared__ uint32_t s_mask[B];
+    __shared__ int s_live[TileWaves<PIX>::count];
     // Per staged Gaussian: the tile's totals of every statistics request.
     __shared__ float s_stat[STATS ? B * RB : 1];
     static_assert(LISTS == 0 || MODE == 0, "capped lists neither count pairs nor total statistics");
@@ -473,32 +559,36 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                 __builtin_nontemporal_store(zero4{0.0f, 0.0f, 0.0f, 0.0f}, z + i);
             if (blockIdx.x == 0 && threadIdx.x < (a.zero_count & 3)) a.zero_out[(n4 << 2) + threadIdx.x] = 0.0f;
         }
-        float fx[PIX], fy[PIX], T[PIX], color[PIX][CH];
-        int px[PIX], py[PIX], last_contributor[PIX];
-        bool done[PIX];
+        // Pixels that have terminated or lie outside the image, as lane masks:
+        // the tests' results meet in scalar registers, beside the vector work.
+        uint64_t done[PIX];
+        float fx[PIX], fy, T[PIX], color[PIX][CH];
+        int px[PIX], py, last_contributor[PIX];
+        bool outside[PIX];
         float val[PIX][STATS ? RB : 1];
         int visited[PIX];
-        uint32_t evaluated = 0, accepted = 0;
+        uint64_t evaluated = 0, accepted = 0;  // of the wavefront
 #pragma unroll
         for (int k = 0; k < PIX; ++k) {
             int lx, ly;
             pixel_of<PIX>(threadIdx.x, k, lx, ly);
             px[k] = t.x0 + lx;
-            py[k] = t.y0 + ly;
+            py = t.y0 + ly;  // a lane's pixels share their row
             fx[k] = (float)px[k];
-            fy[k] = (float)py[k];
-            done[k] = !(px[k] < a.width && py[k] < a.height);
-            visited[k] = done[k] ? 0 : last - t.first;  // the whole list unless the pixel terminates
+            fy = (float)py;
+            outside[k] = !(px[k] < a.width && py < a.height);
+            done[k] = lanes(outside[k]);
+            visited[k] = outside[k] ? 0 : last - t.first;  // the whole list unless the pixel terminates
             T[k] = 1.0f;
             last_contributor[k] = 0;
 #pragma unroll
             for (int c = 0; c < CH; ++c) color[k][c] = 0.0f;
             if constexpr (STATS) {
-                const float* pv = st.pixel_values + t.view * st.pixel_view_stride + (int64_t)py[k] * a.width + px[k];
+                const float* pv = st.pixel_values + t.view * st.pixel_view_stride + (int64_t)py * a.width + px[k];
                 const int64_t plane = (int64_t)a.width * a.height;
 #pragma unroll
                 for (int r = 0; r < RB; ++r) {
-                    const float v = (r < st.requests && !done[k]) ? pv[r * plane] : 0.0f;
+                    const float v = (r < st.requests && !outside[k]) ? pv[r * plane] : 0.0f;
                     // Count requests keep a 0/1 mask (see observe_statistics).
                     val[k][r] = ((st.sum_mask >> r) & 1u) ? v : (v != 0.0f ? 1.0f : 0.0f);
                 }
@@ -529,14 +619,26 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                 for (int r = 0; r < RB; ++r) finite = finite && __builtin_fabsf(val[k][r]) <= 3.0e38f;
             stat_finite = __ballot(!finite) == 0;
         }
+        auto alive = [&]() {
+            uint64_t all = done[0];
+#pragma unroll
+            for (int k = 1; k < PIX; ++k) all &= done[k];
+            return all != ~0ull;
+        };
+        // A barrier that tells whether any wavefront has a live pixel.
+        auto any_alive = [&]() {
+            if (lane == 0) s_live[wave] = alive();
+            __syncthreads();
+            int v = 0;
+#pragma unroll
+            for (int w = 0; w < TileWaves<PIX>::count; ++w) v |= s_live[w];
+            return __builtin_amdgcn_readfirstlane(v) != 0;
+        };
         int stop = -1;  // list entries read before every pixel terminated (-1: never)
         for (int begin = t.first; begin < last; begin += B) {
-            bool active = false;
-#pragma unroll
-            for (int k = 0; k < PIX; ++k) active = active || !done[k];
-            const int active_threads = __syncthreads_count(active);
+            const bool more_pixels = any_alive();
             flush();  // every wavefront is past the previous batch
-            if (active_threads == 0) {
+            if (!more_pixels) {
                 stop = begin - t.first;
                 break;
             }
@@ -546,79 +648,96 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                 if (begin + e < last) {
                     // The 4-channel plain blend fits its registers without the
                     // tile-origin laundering (and is fastest so).
-                    stage_gaussian<CH, PIX, (STATS || CH > 4)>(a, t, g, e, c0, s_g, s_mask);
+                    stage_gaussian<CH, PIX, (STATS || CH > 4)>(a, t, g, e, begin - t.first + e + 1, c0, s_g, s_mask);
                     if constexpr (STATS) flush_id = g;
                 }
                 if (begin + B < last) next_id = a.ids[min(begin + B + e, last - 1)];
             }
             __syncthreads();
             const int cnt = min(B, last - begin);
-            bool live = true;
+            bool live = alive();
             for (int c0 = 0; c0 < cnt && live; c0 += 64) {
                 // This wavefront's Gaussians of the next 64, in list order.
-                uint64_t todo = __ballot(c0 + lane < cnt && ((s_mask[min(c0 + lane, B - 1)] >> wave) & 1u));
+                const uint32_t flags = s_mask[min(c0 + lane, B - 1)];
+                uint64_t todo = lanes(c0 + lane < cnt && ((flags >> wave) & 1u));
                 if (!todo) continue;
+                // Some opacity is not finite (of any of the chunk's Gaussians).
+                const bool strange = (lanes((flags & kStrange) != 0) & todo) != 0;
+                const bool strange_color = (lanes((flags & kStrangeColor) != 0) & todo) != 0;
                 // Blend one Gaussian (batch slot j) into this lane's pixels.
-                auto blend = [&](const Staged<CH>& g, int j) {
-                    const int contributor = begin - t.first + j + 1;  // list position, 1-based
-                    bool acc[PIX];
-                    float wk[PIX];
-                    // Branch-free per pixel except for the exponential: a
-                    // divergent branch per test costs more in exec-mask work than
-                    // the selects it replaces (the wavefront issues the tail
-                    // whenever any lane needs it).  Updates are selected, not
-                    // multiplied by zero, so non-finite features of a rejected
-                    // Gaussian cannot reach the pixel.
+                // Tests are lane masks combined in scalar registers; a pixel
+                // that rejects the Gaussian adds each channel with weight
+                // zero, which leaves a finite sum as it was.  Channels that
+                // are not all finite (FINITE false) are selected instead, so
+                // that a rejected Gaussian's cannot reach the pixel.
+                auto blend = [&](const Staged<CH>& g, int j, auto finite) {
+                    constexpr bool FINITE = decltype(finite)::value;
+                    const float dy = g.xy.y - fy;
+                    const float c_dy_dy = (g.con.z * dy) * dy;
+                    float x[PIX];
+                    uint64_t in[PIX], any = 0;
 #pragma unroll
                     for (int k = 0; k < PIX; ++k) {
-                        const float dx = g.xy.x - fx[k], dy = g.xy.y - fy[k];
-                        const float power = blend_power(g.con.x, g.con.y, g.con.z, dx, dy);
-                        if constexpr (COUNTS) evaluated += done[k] ? 0u : 1u;
-                        const bool in = !done[k] && power <= 0.0f && power >= g.cut;
-                        float e = 0.0f;
-                        if (in) e = blend_exp(power);
-                        const float alpha = in ? sel_min(0.99f, g.con.w * e) : 0.0f;
-                        const bool take = alpha >= 1.0f / 255.0f;
+                        x[k] = blend_exponent(g.con.x, g.con.y, g.xy.x - fx[k], dy, c_dy_dy);
+                        in[k] = lanes(accepts(x[k], g.limit)) & ~done[k];
+                        any |= in[k];
+                        if constexpr (COUNTS) evaluated += __builtin_popcountll(~done[k]);
+                    }
+                    if (!any) return;
+                    if (strange) {
+#pragma unroll
+                        for (int k = 0; k < PIX; ++k) x[k] = clamp_exponent(x[k]);
+                    }
+                    float w[PIX];
+                    uint64_t upd[PIX];
+#pragma unroll
+                    for (int k = 0; k < PIX; ++k) {
+                        const float alpha = sel_min(0.99f, g.con.w * blend_exp_neg(x[k]));
                         const float next_t = T[k] * (1.0f - alpha);
-                        const bool term = take && next_t < 0.0001f;
-                        const bool upd = take && !term;
+                        const uint64_t take = lanes(alpha >= 1.0f / 255.0f) & in[k];
+                        const uint64_t low = lanes(next_t < 0.0001f);
+                        const uint64_t term = take & low;
+                        upd[k] = take & ~low;
+                        done[k] |= term;
+                        w[k] = select0(upd[k], alpha * T[k]);
+                        T[k] = select(upd[k], next_t, T[k]);
                         if constexpr (COUNTS) {
-                            visited[k] = term ? contributor : visited[k];
-                            accepted += upd ? 1u : 0u;
+                            visited[k] = select(term, g.entry, visited[k]);
+                            accepted += __builtin_popcountll(upd[k]);
                         }
-                        done[k] = done[k] || term;
-                        const float w = alpha * T[k];
 #pragma unroll
                         for (int c = 0; c < CH; ++c) {
-                            const float nc = __builtin_fmaf(g.f[c], w, color[k][c]);
-                            color[k][c] = upd ? nc : color[k][c];
+                            const float sum = __builtin_fmaf(g.f[c], w[k], color[k][c]);
+                            color[k][c] = FINITE ? sum : select(upd[k], sum, color[k][c]);
                         }
-                        T[k] = upd ? next_t : T[k];
-                        last_contributor[k] = upd ? contributor : last_contributor[k];
-                        acc[k] = upd;
-                        wk[k] = upd ? w : 0.0f;
+                        last_contributor[k] = select(upd[k], g.entry, last_contributor[k]);
                     }
-
                     if constexpr (STATS) {
-                        bool hit = false;
+                        uint64_t hit = 0;
 #pragma unroll
-                        for (int k = 0; k < PIX; ++k) hit = hit || acc[k];
-                        if (__ballot(hit))
-                            observe_statistics<PIX, RB, KINDS>(st, stat_r, &s_stat[j * RB], acc, wk, val, stat_finite, lane);
+                        for (int k = 0; k < PIX; ++k) hit |= upd[k];
+                        if (hit)
+                            observe_statistics<PIX, RB, KINDS>(st, stat_r, &s_stat[j * RB], upd, w, val, stat_finite, lane);
                     }
-                };
-                auto alive = [&]() {
-                    bool any = false;
-#pragma unroll
-                    for (int k = 0; k < PIX; ++k) any = any || !done[k];
-                    return __ballot(any) != 0;
                 };
                 auto take = [&]() {
                     const int j = c0 + __builtin_ctzll(todo);
                     todo &= todo - 1;
                     return j;
                 };
-                if constexpr ((STATS && (RB > 2 || CH > 4)) || (CH > 16 && CH <= 36)) {
+                auto at_use = [&](auto finite) {
+                    while (todo) {
+                        if (!alive()) {
+                            live = false;
+                            break;
+                        }
+                        const int j = take();
+                        blend(load_staged<CH>(j, s_g), j, finite);
+                    }
+                };
+                if (strange_color) {
+                    at_use(std::false_type{});
+                } else if constexpr ((STATS && (RB > 2 || CH > 4)) || (CH > 16 && CH <= 36)) {
                     // Loads at use: the pipelined form's extra registers would
                     // cost occupancy -- with statistics beyond two requests (their
                     // pixel values take 4 * PIX registers or more) or four
@@ -627,14 +746,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                     // channels a third wavefront per SIMD (148 VGPRs against 190
                     // with the next Gaussian's vector prefetched: 0.83 -> 0.72
                     // ms on the 32-feature workload).
-                    while (todo) {
-                        if (!alive()) {
-                            live = false;
-                            break;
-                        }
-                        const int j = take();
-                        blend(load_staged<CH>(j, s_g), j);
-                    }
+                    at_use(std::true_type{});
                 } else {
                     // Unrolled by two: the next Gaussian is loaded into the other
                     // buffer before the current one is blended.
@@ -650,19 +762,17 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                             jb = take();
                             gb = load_staged<CH>(jb, s_g);
                         }
-                        blend(ga, ja);
+                        blend(ga, ja, std::true_type{});
                         if (!more) break;
                         // Liveness is checked once per two Gaussians: a Gaussian
                         // blended after every pixel is done changes nothing (no
-                        // pixel accepts it), and the check costs VALU and scalar
-                        // work on every Gaussian (1091 -> 1067 us for the
-                        // 3M-Gaussian forward blend).
+                        // pixel accepts it).
                         more = todo != 0;
                         if (more) {
                             ja = take();
                             ga = load_staged<CH>(ja, s_g);
                         }
-                        blend(gb, jb);
+                        blend(gb, jb, std::true_type{});
                         if (!more) break;
                     }
                 }
@@ -676,10 +786,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
         if constexpr (LISTS != 0) {
             if (stop < 0) {
                 // The loop ran to the end of the list it had: all of it read.
-                bool active = false;
-#pragma unroll
-                for (int k = 0; k < PIX; ++k) active = active || !done[k];
-                if (__syncthreads_count(active) == 0) stop = last - t.first;
+                if (!any_alive()) stop = last - t.first;
             }
             if (threadIdx.x == 0 && c0 == 0) {
                 // A capped tile with pixels still live needs its whole list:
@@ -702,8 +809,8 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
         const int F = a.feat_channels, E = a.extra_channels;
 #pragma unroll
         for (int k = 0; k < PIX; ++k) {
-            if (!(px[k] < a.width && py[k] < a.height)) continue;
-            const int64_t pix = ((int64_t)t.view * a.height + py[k]) * a.width + px[k];
+            if (outside[k]) continue;
+            const int64_t pix = ((int64_t)t.view * a.height + py) * a.width + px[k];
 #pragma unroll
             for (int c = 0; c < CH; ++c) {
                 const int gc = c0 + c;
@@ -725,13 +832,9 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
             uint64_t v = 0;
 #pragma unroll
             for (int k = 0; k < PIX; ++k) v += (uint64_t)visited[k];
-            uint64_t e = evaluated, c = accepted;
+            const uint64_t e = evaluated, c = accepted;
 #pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) {
-                v += (uint64_t)__shfl_xor((long long)v, d, 64);
-                e += (uint64_t)__shfl_xor((long long)e, d, 64);
-                c += (uint64_t)__shfl_xor((long long)c, d, 64);
-            }
+            for (int d = 32; d >= 1; d >>= 1) v += (uint64_t)__shfl_xor((long long)v, d, 64);
             if (lane == 0) {
                 atomicAdd(counts, (unsigned long long)v);
                 atomicAdd(counts + 1, (unsigned long long)e);
@@ -939,7 +1042,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                 // Tile origin laundered (see stage_gaussian): 75 instead of
                 // 79 VGPRs, no spill with absolute gradients, 1.7% faster
                 // at 36 channels.
-                stage_gaussian<CH, PIX, true>(a, t, g, e, c0, s_g, s_mask);
+                stage_gaussian<CH, PIX, true>(a, t, g, e, p + 1, c0, s_g, s_mask);
             }
             if (top > B) next_id = a.ids[t.first + max(p - B, 0)];
         }
@@ -958,7 +1061,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
             if (__ballot(pos < lane_last) == 0) continue;
             const float2 xy = s_g[j].xy;
             const float4 con = s_g[j].con;
-            const float cut = s_g[j].cut;
+            const float limit = s_g[j].limit;
             const float* f = s_g[j].f;
             // Accumulators start from an opaque zero: a literal zero would be
             // folded into each accumulator's first FMA, and every path that
@@ -978,7 +1081,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                 if (!(pos < last_contributor[k])) continue;
                 const float dx = xy.x - fx[k], dy = xy.y - fy[k];
                 const float power = blend_power(con.x, con.y, con.z, dx, dy);
-                if (!(power <= 0.0f) || !(power >= cut)) continue;
+                if (!(power <= 0.0f) || !(power >= -limit)) continue;
                 const float G = blend_exp(power);
                 const float og = con.w * G;
                 const float alpha = sel_min(0.99f, og);
