@@ -2,25 +2,30 @@
 //
 // gs3d/render.py:36-208 (forward) and :211-356 (backward).  One workgroup
 // per tile.  A lane owns PIX pixels of the tile (1: one pixel, 256 threads;
-// 2: a horizontal pair, 128 threads; 4: a 2x2 quad, 64 threads = one
-// wavefront for the whole tile).  The tile's sorted Gaussians are staged in
-// LDS in batches (centre, conic + opacity, exponent cutoff and the full
+// 2: a horizontal pair, 128 threads).  The tile's sorted Gaussians are staged
+// in LDS in batches (centre, conic + opacity, exponent limit and the full
 // blended channel vector), so the inner loop reads only LDS broadcasts.  A
-// lane leaves the inner loop once its pixels are done, a wavefront once its
-// lanes are, and the workgroup stops at the next batch once all pixels are.
+// wavefront leaves the inner loop once its pixels are done, and the workgroup
+// stops at the next batch once all pixels are.
 //
-// Exponent cutoff: a Gaussian with opacity o can only reach alpha >= 1/255
-// where power >= -ln(255 o); below that bound minus a 1% margin (far above
+// Exponent limit: a Gaussian with opacity o can only reach alpha >= 1/255
+// where -power <= ln(255 o); beyond that bound plus a 1% margin (far above
 // the few-ulp error of exp, log and the product) the blend rejects the
-// Gaussian without evaluating exp.  Decisions, and therefore every output,
-// are identical to evaluating it.
+// Gaussian.  Decisions, and therefore every output, are identical to
+// evaluating the exponential.
 //
-// Backward: every lane accumulates its pixels' contributions to the current
-// Gaussian; the wavefront sums all gradient entries together (permlane swaps
-// pair the entries, a DPP row butterfly finishes them) and one atomic
+// Vector arithmetic bounds both directions.  Measured per SIMD with several
+// wavefronts: 2.7 cycles for a float add, multiply or fused multiply-add, 4.5
+// for a compare, select, conversion, ldexp or DPP add, 8.5 for a reciprocal or
+// a permlane swap, and 23 for a two-operand select on vcc right behind
+// another.  So the loops keep their tests as scalar lane masks, form the
+// exponential from adds, multiplies and one shift, and add a rejected
+// Gaussian's channels with weight zero instead of selecting each sum.
+//
+// Backward: only batches below the largest last contributor of the tile are
+// visited; a wavefront sums its pixels' gradients before one atomic
 // instruction adds them, one entry per lane, instead of one atomic per entry
-// and pixel as in the reference.  Only batches below the largest last contributor of the
-// tile are visited.
+// and pixel as in the reference.
 //
 // Channel windows: the reference specialises its kernels on any channel count
 // D' (gs3d/render.py:36-38, :211-213).  A launch here blends a window of at
@@ -497,9 +502,11 @@ GS3D_DEV void observe_statistics(const gs3d_render_stats_args& st, int dst_r, fl
     if (dst_r >= 0 && total != 0.0f) atomicAdd(slot + dst_r, total);  // LDS
 }
 
-// Up to 8 channels the kernel is held to 80 VGPRs (6 wavefronts per SIMD
-// instead of 5: 1.180 -> 1.130 ms on RGB); wider channel vectors keep the
-// registers they need.
+// Up to 4 channels the kernel is held to 80 VGPRs (6 wavefronts per SIMD
+// instead of 5: 1.180 -> 1.130 ms on RGB), up to 8 to 96, up to 36 to 168 (3
+// wavefronts).  Lane masks, weights of zero and the exponential from adds
+// (see the file comment): 3M Gaussians, 4 x 1920x1080, 1005 -> 790 us; 500K
+// at 1280x720 169 -> 138 us; 34 channels at 1600x1200 688 -> 596 us.
 //
 // MODE: 0 plain; 1 with contribution statistics; 2 also counting (pixel,
 // Gaussian) pairs into counts[0..2]: visited as the reference's loop visits
@@ -882,15 +889,491 @@ GS3D_DEV float rest_dot(const gs3d_render_bwd_args& b, int view, int64_t g, floa
     return dot;
 }
 
-// Four channels fit 80 VGPRs, six wavefronts per SIMD (the LDS limit of a
-// 13 KiB block); with absolute gradients the uncapped allocation is 83.
+// ---------------------------------------------------------------------------
+// Backward, up to 16 channels: four Gaussians at a time
+//
+// The gradients of a Gaussian are sums over pixels that depend on a pixel
+// through two numbers, the blend weight alpha T (colour gradients) and
+// h = e^power dL/dalpha (everything else: with w = o h the centre gradient is
+// -sum w (a dx + b dy, c dy + b dx), the conic's -1/2 sum w (dx dx, 2 dx dy,
+// dy dy), the opacity's sum h).  So a lane keeps only those two per pixel, for
+// four accepted Gaussians; eight or sixteen permlane swaps then exchange them
+// such that the 16 lanes of row q hold Gaussian q, each lane with the pixels of
+// four of the wavefront's row pairs.  There the sums over a lane's pixels are
+// separable moments -- over its pixels h, h dy and h dy dy need no product
+// with dx per pixel -- and one reduction over 16 lanes finishes four
+// Gaussians, whose entries one atomic instruction adds.  Before, every
+// Gaussian's ten products were formed per pixel and summed over 64 lanes by
+// themselves, 40% of the kernel's vector time.
+// ---------------------------------------------------------------------------
+
+// Exchanges register r's row s of 16 lanes with register s's row r, for two
+// sets of four registers.  In one block: the wait states that a swap needs
+// after a vector write of its operands are spelled out once, and between the
+// two levels the other set's swaps provide them.
+GS3D_DEV void exchange_rows(float (&a)[4], float (&b)[4]) {
+    asm volatile(
+        "s_nop 1\n\t"
+        "v_permlane32_swap_b32 %0, %2\n\t"
+        "v_permlane32_swap_b32 %1, %3\n\t"
+        "v_permlane32_swap_b32 %4, %6\n\t"
+        "v_permlane32_swap_b32 %5, %7\n\t"
+        "v_permlane16_swap_b32 %0, %1\n\t"
+        "v_permlane16_swap_b32 %2, %3\n\t"
+        "v_permlane16_swap_b32 %4, %5\n\t"
+        "v_permlane16_swap_b32 %6, %7\n\t"
+        "s_nop 1"
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
+}
+
+// Sums V values over each row of 16 lanes; for every i the total of value
+// 4 * i + row_bank_value(lane) ends in v[4 * i] of every lane.  The first
+// two levels write two values' sums into the two halves, then the four banks
+// of four lanes, of one register (masked DPP adds): 21 instructions for ten
+// values.  Each block starts with the wait states a DPP read needs.
+template <int V>
+GS3D_DEV void sum_rows_packed(float (&v)[V]) {
+#pragma unroll
+    for (int i = 0; i < V; i += 2) {
+        if (i + 1 < V)
+            asm volatile(
+                "s_nop 1\n\t"
+                "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+                "v_add_f32_dpp %0, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xc"
+                : "+v"(v[i]) : "v"(v[i + 1 < V ? i + 1 : i]));
+        else
+            asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf" : "+v"(v[i]));
+    }
+#pragma unroll
+    for (int i = 0; i < V; i += 4) {
+        if (i + 2 < V)
+            asm volatile(
+                "s_nop 1\n\t"
+                "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                "v_add_f32_dpp %0, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xa"
+                : "+v"(v[i]) : "v"(v[i + 2 < V ? i + 2 : i]));
+        else
+            asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf" : "+v"(v[i]));
+    }
+#pragma unroll
+    for (int i = 0; i < V; i += 4)
+        asm volatile(
+            "s_nop 1\n\t"
+            "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 1\n\t"
+            "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
+            : "+v"(v[i]));
+}
+
+GS3D_DEV int row_bank_value(int lane) {
+    const int bank = (lane >> 2) & 3;
+    return 2 * (bank & 1) + (bank >> 1);
+}
+
+// a x + b y to about one rounding of its own value: the rounding error of
+// b y, which dominates where the terms cancel, is added back.
+GS3D_DEV float dot2_accurate(float a, float x, float b, float y) {
+    const float p = b * y;
+    const float e = __builtin_fmaf(b, y, -p);
+    return __builtin_fmaf(a, x, p) + e;
+}
+
+// Upstream gradient of blended channel gc at pixel index pix.
+GS3D_DEV float upstream_at(const gs3d_render_bwd_args& b, int64_t pix, int gc, int D) {
+    // The channel's source (wave-uniform selects, no branch); channels
+    // without one read final_t and take 0.
+    const int F = b.fwd.feat_channels, E = b.fwd.extra_channels;
+    const float* src = gc < F ? b.upstream : gc < F + E ? b.upstream_extra : b.upstream_alpha;
+    const int64_t stride = gc < F ? b.upstream_stride : gc < F + E ? b.upstream_extra_stride : b.upstream_alpha_stride;
+    const int off = gc < F ? gc : gc < F + E ? gc - F : 0;
+    const bool has = gc < D && src != nullptr;
+    const float u = has ? src[pix * stride + off] : b.fwd.final_t[pix];
+    return has ? u : 0.0f;
+}
+
+// D <= CH channels, of which at most NC have gradients (the constant alpha
+// channel, last, has none).  Bound by vector instructions: at two pixels per
+// lane about 90 per Gaussian undo it from the pixels and 35 are its share of a
+// group's sums; without the atomics the kernel takes 1% less where Gaussians
+// are small and 24% less where some cover thousands of tiles.  3M Gaussians,
+// 4 x 1920x1080: 1640 -> 1455 us (94 VGPRs, five wavefronts per SIMD); 500K at
+// 1280x720 with absolute gradients 304 -> 227 us; 78K at 637x421 with 9
+// channels 238 -> 177 us.  The pixels' gradients for the second half lie in LDS: in registers
+// (24 more) the kernel spilled or lost a wavefront per SIMD.
+// Gaussians staged per batch: the staged channels and the pixels' gradients
+// share the LDS that resident workgroups leave.
+template <int CH>
+struct RowsBatch {
+    static constexpr int size = CH <= 8 ? 128 : CH <= 16 ? 256 : 64;
+};
+
+template <int CH, int NC, bool ABS, int PIX>
+__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 5 : CH <= 16 ? 4 : 3))) void render_bwd_rows_kernel(gs3d_render_bwd_args b) {
+    constexpr int NT = kTilePixels / PIX;
+    constexpr int B = RowsBatch<CH>::size;
+    constexpr int FB = ABS ? 8 : 6;
+    constexpr int V = FB + NC;  // entries: centre xy, conic abc, opacity, [|centre| xy], channels
+    constexpr int ATOMICS = (V + 15) / 16;
+    static_assert(B <= 256, "four batch slots are packed into one word");
+    static_assert(B <= NT, "one staged Gaussian per thread and batch");
+    static_assert(NC == CH || NC == CH - 1, "");
+    __shared__ StagedRec<CH> s_g[B];
+    __shared__ uint32_t s_mask[B];
+    __shared__ int32_t s_id[B];
+    __shared__ int s_max_last;
+    // The wavefronts' upstream gradients by place after the exchange: [row
+    // pair and pixel of the lane][lane of the row of 16].
+    struct alignas(16) PixelGrad {
+        float c[(NC + 3) / 4 * 4];  // the padding may be read, never used
+    };
+    __shared__ PixelGrad s_grad[TileWaves<PIX>::count][4 * PIX][16];
+    const gs3d_render_args& a = b.fwd;
+    const TileInfo t = tile_info(a);
+    const int F = a.feat_channels, E = a.extra_channels;
+    const int D = F + E + (a.one_tail ? 1 : 0);
+    const int lane = lane_id(), wave = threadIdx.x >> 6, q = lane >> 4;
+    // Per pixel: S = sum_c accum_c * grad_c, the colour accumulated behind
+    // the current Gaussian dotted with the upstream gradient.  With
+    // dot = sum_c f_c * grad_c the alpha gradient sum_c (f_c - accum_c) grad_c
+    // (gs3d/render.py:300-312) is E = dot - S, and
+    // accum_c = la last_c + (1 - la) accum_c becomes S = S + la E_last with
+    // la and E_last those of the last accepted Gaussian: no per-channel state
+    // besides grad.  bg_t = -T_final * sum_c bg_c grad_c is the background
+    // term, divided by the transmittance factors as they are undone.
+    float fx[PIX], fy, T[PIX], bg_t[PIX], last_alpha[PIX], S[PIX], last_e[PIX];
+    float grad[PIX][CH];
+    int last_contributor[PIX];
+    bool inside[PIX];
+    if (threadIdx.x == 0) s_max_last = 0;
+    const float* bg = a.background ? a.background + t.view * a.background_view_stride : nullptr;
+    int my_max = 0;
+    int x_first, y_own;
+    pixel_of<PIX>(threadIdx.x, 0, x_first, y_own);
+    x_first += t.x0;
+    y_own += t.y0;
+    fy = (float)y_own;
+    auto pixel_index = [&](int x, int y) {
+        return ((int64_t)t.view * a.height + min(y, a.height - 1)) * a.width + min(x, a.width - 1);
+    };
+    // Per-pixel inputs: every load first, from the pixel clamped into the
+    // image, then the pixels outside the image are cleared.  A load under a
+    // per-lane condition would be a branch that waits for its data.
+#pragma unroll
+    for (int k = 0; k < PIX; ++k) {
+        const int64_t pix = pixel_index(x_first + k, y_own);
+        fx[k] = (float)(x_first + k);
+        inside[k] = x_first + k < a.width && y_own < a.height;
+        T[k] = a.final_t[pix];
+        last_contributor[k] = a.contributors[pix];
+#pragma unroll
+        for (int c = 0; c < CH; ++c) grad[k][c] = upstream_at(b, pix, c, D);
+    }
+    bool finite = true;
+#pragma unroll
+    for (int k = 0; k < PIX; ++k) {
+        bg_t[k] = last_alpha[k] = S[k] = last_e[k] = 0.0f;
+        if (!inside[k]) {
+            T[k] = 0.0f;
+            last_contributor[k] = 0;
+#pragma unroll
+            for (int c = 0; c < CH; ++c) grad[k][c] = 0.0f;
+        }
+        PixelGrad& place = s_grad[wave][PIX * q + k][lane & 15];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            place.c[c] = grad[k][c];
+            finite = finite && __builtin_fabsf(grad[k][c]) <= 3.4028235e38f;
+        }
+        float bg_grad = 0.0f;
+        if (bg) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) bg_grad += (c < F ? bg[c] : 0.0f) * grad[k][c];
+        }
+        if (inside[k]) bg_t[k] = -T[k] * bg_grad;
+        my_max = max(my_max, last_contributor[k]);
+    }
+    const bool all_finite = lanes(!finite) == 0;
+    __syncthreads();
+    if (my_max > 0) atomicMax(&s_max_last, my_max);
+    __syncthreads();
+    const int max_last = min(s_max_last, t.last - t.first);
+    // The gradient entries this lane adds for its row's Gaussian, one per
+    // atomic instruction: an entry of Gaussian g lies at base + g * step.
+    struct Destination {
+        float* base;
+        uint32_t step;  // row strides below 2^31 (checked on the host)
+        float scale;
+        bool times_opacity;
+    } dst[ATOMICS];
+#pragma unroll
+    for (int i = 0; i < ATOMICS; ++i) {
+        const int k = 4 * (4 * i + (lane & 3)) + row_bank_value(lane);
+        const int64_t row0 = (int64_t)t.view * a.n;
+        Destination d = {nullptr, 0, 1.0f, k < FB && k != 5};
+        if (k < 2 || k == 3) d.scale = -1.0f;
+        if (k == 2 || k == 4) d.scale = -0.5f;
+        if (k >= V) {
+        } else if (k < 2) {
+            d.base = b.grad_centers + row0 * b.grad_centers_stride + k;
+            d.step = b.grad_centers_stride;
+        } else if (k < 6) {
+            d.base = b.grad_conics + row0 * b.grad_conics_stride + (k - 2);
+            d.step = b.grad_conics_stride;
+        } else if (ABS && k < 8) {
+            d.base = b.abs_centers + row0 * b.abs_stride + (k - 6);
+            d.step = b.abs_stride;
+        } else {
+            const int c = k - FB;
+            if (c < F) {
+                if (b.grad_features) {
+                    d.base = b.grad_features + t.view * b.grad_feat_view_stride + c;
+                    d.step = b.grad_feat_stride;
+                }
+            } else if (c < F + E && b.grad_extra) {
+                d.base = b.grad_extra + t.view * b.grad_extra_view_stride + (c - F);
+                d.step = b.grad_extra_stride;
+            }
+        }
+        dst[i] = d;
+    }
+    // Largest last contributor among this wavefront's pixels (wave-uniform).
+    int wave_last = my_max;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) wave_last = max(wave_last, __shfl_xor(wave_last, d, 64));
+    // As in the forward: one staged Gaussian per thread and batch, its index
+    // for the next batch loaded while the current one is traversed.
+    int32_t next_id = max_last > 0 ? a.ids[t.first + max(max_last - 1 - (int)threadIdx.x, 0)] : 0;
+    for (int top = max_last; top > 0; top -= B) {
+        __syncthreads();
+        if (threadIdx.x < B) {
+            const int e = threadIdx.x;
+            const int p = top - 1 - e;
+            const int32_t g = next_id;
+            if (p >= 0) {
+                s_id[e] = g;
+                stage_gaussian<CH, PIX, true>(a, t, g, e, p + 1, 0, s_g, s_mask);
+            }
+            if (top > B) next_id = a.ids[t.first + max(p - B, 0)];
+        }
+        __syncthreads();
+        const int cnt = min(B, top);
+        // Up to four blended Gaussians: values [pixel][slot], and their batch
+        // slots, a byte each.
+        float aT[PIX][4], h[PIX][4];
+        uint32_t slots = 0;
+        int used = 0;
+        // The gradients of the Gaussians in the slots.
+        auto finish = [&]() {
+                            // Row q of lanes: Gaussian q of the four, [pixel][row pair].
+            #pragma unroll
+                            for (int k = 0; k < PIX; ++k) exchange_rows(aT[k], h[k]);
+                            const int j = (slots >> (8 * q)) & 255;
+                            const float4 con = s_g[j].con;
+                            const float2 xy = s_g[j].xy;
+                            const int32_t id = s_id[j];
+                            float dx[PIX], dy[4];
+            #pragma unroll
+                            for (int k = 0; k < PIX; ++k) dx[k] = xy.x - fx[k];
+            #pragma unroll
+                            for (int r = 0; r < 4; ++r) dy[r] = (xy.y - (fy - (float)(2 * q))) - (float)(2 * r);
+                            float v[V];
+                            // Moments over the lane's pixels: per column k the sums of h
+                            // and h dy, per row pair P_r = sum_k h.
+                            float A[PIX], H[PIX], P[4], yy = 0.0f;
+            #pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                P[r] = PIX == 2 ? h[0][r] + h[PIX - 1][r] : h[0][r];
+                                const float py = P[r] * dy[r];
+                                yy = r ? __builtin_fmaf(py, dy[r], yy) : py * dy[r];
+                            }
+            #pragma unroll
+                            for (int k = 0; k < PIX; ++k) {
+                                A[k] = (h[k][0] + h[k][1]) + (h[k][2] + h[k][3]);
+                                H[k] = h[k][0] * dy[0];
+            #pragma unroll
+                                for (int r = 1; r < 4; ++r) H[k] = __builtin_fmaf(h[k][r], dy[r], H[k]);
+                            }
+                            const float mass = PIX == 2 ? A[0] + A[PIX - 1] : A[0];
+                            // The centre gradient from the moments about the middle of
+                            // the lane's pixels (column offsets of 1/2, rows of 1 and 3):
+                            // a dx + b dy may cancel, and is taken there to one rounding.
+                            const float mx = PIX == 2 ? 0.5f * (A[0] - A[PIX - 1]) : 0.0f;
+                            const float my = __builtin_fmaf(3.0f, P[0] - P[3], P[1] - P[2]);
+                            const float dxm = PIX == 2 ? dx[0] - 0.5f : dx[0], dym = dy[0] - 3.0f;
+                            const float ux = dot2_accurate(con.x, dxm, con.y, dym);
+                            const float uy = dot2_accurate(con.z, dym, con.y, dxm);
+                            v[0] = __builtin_fmaf(ux, mass, con.y * my);
+                            v[1] = __builtin_fmaf(uy, mass, con.z * my);
+                            if constexpr (PIX == 2) {
+                                v[0] = __builtin_fmaf(con.x, mx, v[0]);
+                                v[1] = __builtin_fmaf(con.y, mx, v[1]);
+                            }
+                            v[2] = (A[0] * dx[0]) * dx[0];
+                            v[3] = H[0] * dx[0];
+                            if constexpr (PIX == 2) {
+                                v[2] = __builtin_fmaf(A[PIX - 1] * dx[PIX - 1], dx[PIX - 1], v[2]);
+                                v[3] = __builtin_fmaf(H[PIX - 1], dx[PIX - 1], v[3]);
+                            }
+                            v[4] = yy;
+                            v[5] = mass;
+                            if constexpr (ABS) {
+                                v[6] = v[7] = 0.0f;
+            #pragma unroll
+                                for (int r = 0; r < 4; ++r) {
+                                    const float bdy = con.y * dy[r], cdy = con.z * dy[r];
+            #pragma unroll
+                                    for (int k = 0; k < PIX; ++k) {
+                                        const float px = __builtin_fmaf(con.x, dx[k], bdy), py = __builtin_fmaf(con.y, dx[k], cdy);
+                                        v[6] = __builtin_fmaf(__builtin_fabsf(h[k][r]), __builtin_fabsf(px), v[6]);
+                                        v[7] = __builtin_fmaf(__builtin_fabsf(h[k][r]), __builtin_fabsf(py), v[7]);
+                                    }
+                                }
+                            }
+                            // A pixel that did not blend the Gaussian has weight zero; a
+            // non-finite gradient there must not reach it.
+            // The widest vectors' gradients do not fit the registers together:
+            // four channels of all pixels at a time.
+            constexpr int CG = NC > 16 ? 4 : NC;
+#pragma unroll
+            for (int c0 = 0; c0 < NC; c0 += CG) {
+                if constexpr (CG < NC) asm volatile("" ::: "memory");
+                float sum[CG];
+#pragma unroll
+                for (int c = 0; c < CG; ++c) sum[c] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 4 * PIX; ++i) {
+                    alignas(16) float u[(CG + 3) / 4 * 4];
+#pragma unroll
+                    for (int c = 0; c < CG; c += 4)
+                        *reinterpret_cast<float4*>(u + c) =
+                            *reinterpret_cast<const float4*>(s_grad[wave][i][lane & 15].c + c0 + c);
+                    const float w = aT[i % PIX][i / PIX];
+                    if (all_finite) {
+#pragma unroll
+                        for (int c = 0; c < CG; ++c) sum[c] = __builtin_fmaf(w, u[c], sum[c]);
+                    } else {
+#pragma unroll
+                        for (int c = 0; c < CG; ++c) sum[c] += w != 0.0f ? w * u[c] : 0.0f;
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < CG; ++c)
+                    if (c0 + c < NC) v[FB + (c0 + c < NC ? c0 + c : 0)] = sum[c];
+            }
+            sum_rows_packed<V>(v);
+            #pragma unroll
+                            for (int i = 0; i < ATOMICS; ++i) {
+                                float total = v[16 * i];
+            #pragma unroll
+                                for (int m = 1; m < 4; ++m)
+                                    if (16 * i + 4 * m < V) total = ((lane & 3) == m) ? v[16 * i + 4 * m] : total;
+                                total *= dst[i].times_opacity ? dst[i].scale * con.w : dst[i].scale;
+                                // One 32 x 32 -> 64-bit multiply-add for the address (ids
+                                // are non-negative, strides below 2^31).
+                                if (dst[i].base && q < used)
+                                    atomicAdd(dst[i].base + (uint64_t)(uint32_t)id * dst[i].step, total);
+                            }
+                            used = 0;
+                            slots = 0;
+        };
+        for (int c0 = 0; c0 < cnt; c0 += 64) {
+            // This wavefront's Gaussians of the next 64 that lie before its
+            // pixels' last contributors, in traversal order.
+            const int slot0 = c0 + lane;
+            const uint32_t flags = s_mask[min(slot0, B - 1)];
+            uint64_t todo = lanes(slot0 < cnt && top - 1 - slot0 < wave_last && ((flags >> wave) & 1u));
+            const bool strange = (lanes((flags & kStrange) != 0) & todo) != 0;
+            while (todo) {
+                // One Gaussian undone from this lane's pixels: its weight and h.
+                const int j = c0 + __builtin_ctzll(todo);
+                todo &= todo - 1;
+                const Staged<CH> g = load_staged<CH>(j, s_g);
+                const int entry = top - j;  // list position, 1-based
+                const float dy = g.xy.y - fy;
+                const float c_dy_dy = (g.con.z * dy) * dy;
+                float x[PIX];
+                uint64_t in[PIX], any = 0;
+#pragma unroll
+                for (int k = 0; k < PIX; ++k) {
+                    x[k] = blend_exponent(g.con.x, g.con.y, g.xy.x - fx[k], dy, c_dy_dy);
+                    in[k] = lanes(accepts(x[k], g.limit)) & lanes(entry <= last_contributor[k]);
+                    any |= in[k];
+                }
+                if (!any) continue;
+                float G[PIX], alpha[PIX], weight[PIX], hv[PIX];
+                if (strange) {
+#pragma unroll
+                    for (int k = 0; k < PIX; ++k) G[k] = blend_exp(-x[k]);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < PIX; ++k) G[k] = blend_exp_neg(x[k]);
+                }
+                any = 0;
+#pragma unroll
+                for (int k = 0; k < PIX; ++k) {
+                    alpha[k] = sel_min(0.99f, g.con.w * G[k]);
+                    in[k] &= lanes(alpha[k] >= 1.0f / 255.0f);
+                    any |= in[k];
+                }
+                if (!any) continue;
+#pragma unroll
+                for (int k = 0; k < PIX; ++k) {
+                    // Gradients only need tolerance-level agreement: one hardware
+                    // reciprocal (1 - alpha >= 0.01) and fused multiply-adds.
+                    const float inv = __builtin_amdgcn_rcpf(1.0f - alpha[k]);
+                    // Channel slots at or beyond D hold zero features and
+                    // zero upstream gradients; a last slot without a
+                    // gradient is the constant channel or one of those.
+                    float dot = NC < CH ? grad[k][CH - 1] : g.f[CH - 1] * grad[k][CH - 1];
+#pragma unroll
+                    for (int c = 0; c + 1 < CH; ++c) dot = __builtin_fmaf(g.f[c], grad[k][c], dot);
+                    // A branch: the pixel's state then changes in place.
+                    if (__builtin_amdgcn_inverse_ballot_w64(in[k])) {
+                        T[k] = T[k] * inv;
+                        S[k] = __builtin_fmaf(last_alpha[k], last_e[k], S[k]);
+                        last_e[k] = dot - S[k];
+                        last_alpha[k] = alpha[k];
+                    }
+                    weight[k] = alpha[k] * T[k];
+                    hv[k] = G[k] * __builtin_fmaf(last_e[k], T[k], bg_t[k] * inv);
+                }
+                // Into the next slot (a wave-uniform branch).
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    if (used == s) {
+#pragma unroll
+                        for (int k = 0; k < PIX; ++k) {
+                            aT[k][s] = select0(in[k], weight[k]);
+                            h[k][s] = select0(in[k], hv[k]);
+                        }
+                    }
+                slots |= (uint32_t)j << (8 * used);
+                if (++used == 4) finish();
+            }
+        }
+        if (used) {
+            // The slots past the last one.
+#pragma unroll
+            for (int s = 1; s < 4; ++s)
+                if (used <= s) {
+#pragma unroll
+                    for (int k = 0; k < PIX; ++k) aT[k][s] = h[k][s] = 0.0f;
+                }
+            finish();
+        }
+    }
+}
+
+// The backward of wider vectors, one Gaussian at a time: every lane
+// accumulates its pixels' contributions to the current Gaussian and the
+// wavefront sums all entries together (wave_sum_rows).
 //
 // GEOM: the geometry launch (window 0, c0 = 0): centre, conic and opacity
 // gradients (+ absolute centre gradients with ABS) and the window's feature
 // gradients; channels from CH on, if any, enter the alpha gradient through
 // rest_dot.  !GEOM: a further window [c0, c0 + CH), feature gradients only.
 template <int CH, bool ABS, int PIX, bool GEOM>
-__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 6 : 1))) void render_bwd_kernel(gs3d_render_bwd_args b, int c0) {
+__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(1))) void render_bwd_kernel(gs3d_render_bwd_args b, int c0) {
     constexpr int NT = kTilePixels / PIX;
     constexpr int B = Batch<CH>::size;
     // Gradient entries per Gaussian: [centre xy, conic abc, opacity, |centre| xy]
@@ -1160,10 +1643,12 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
 // small frame still spreads over the SIMDs.  Each tile's list is walked
 // serially; at two pixels per lane a few thousand tiles make little more than
 // one full set of resident wavefronts (6 per SIMD, 6144 on the chip), and the
-// longest lists set the time (500K Gaussians at 1280x720, 3600 tiles: a step 0.93 ->
-// 0.87 ms at one pixel per lane; 1920x1080, 8160 tiles: 1.31 -> 1.64 ms).
+// longest lists set the time.  Forward and backward at one against two pixels
+// per lane: three 801x601 views (5814 tiles) 281 + 474 against 323 + 569 us;
+// 1920x1080 with very large Gaussians (8160 tiles) 312 + 1169 against 289 +
+// 733 us; two 1920x1080 views (16320 tiles) 389 + 800 against 367 + 672 us.
 #ifndef GS3D_SMALL_GRID
-#define GS3D_SMALL_GRID 4096
+#define GS3D_SMALL_GRID 6144
 #endif
 constexpr unsigned kSmallGrid = GS3D_SMALL_GRID;
 // Workgroups of a redo launch (gs3d_render_args.redo_pass).
@@ -1233,25 +1718,42 @@ inline int launch_fwd_window(const gs3d_render_args& a, const gs3d_render_stats_
     return launch_fwd<kWindow>(a, st, counts, blocks, c0, s);
 }
 
-template <int CH, bool GEOM, int PIX>
-int launch_bwd_pix(const gs3d_render_bwd_args& b, unsigned blocks, int c0, hipStream_t s) {
-    if constexpr (GEOM) {
-        if (b.abs_centers) {
-            hipLaunchKernelGGL((render_bwd_kernel<CH, true, PIX, true>), dim3(blocks), dim3(kTilePixels / PIX), 0, s, b, c0);
-            return launch_status("gs3d_render_bwd");
-        }
-    }
-    hipLaunchKernelGGL((render_bwd_kernel<CH, false, PIX, GEOM>), dim3(blocks), dim3(kTilePixels / PIX), 0, s, b, c0);
+template <int CH, int NC, int PIX>
+int launch_bwd_rows(const gs3d_render_bwd_args& b, unsigned blocks, hipStream_t s) {
+    const dim3 grid(blocks), block(kTilePixels / PIX);
+    if (b.abs_centers)
+        hipLaunchKernelGGL((render_bwd_rows_kernel<CH, NC, true, PIX>), grid, block, 0, s, b);
+    else
+        hipLaunchKernelGGL((render_bwd_rows_kernel<CH, NC, false, PIX>), grid, block, 0, s, b);
     return launch_status("gs3d_render_bwd");
+}
+
+// All gradients of a vector of at most 16 channels.
+template <int CH>
+int launch_bwd_rows(const gs3d_render_bwd_args& b, unsigned blocks, int gradient_channels, hipStream_t s) {
+    constexpr int PIX = PixFor<CH, true>::value;
+    auto run = [&](auto nc) {
+        constexpr int NC = decltype(nc)::value;
+        if constexpr (PIX > 1) {
+            if (blocks < kSmallGrid) return launch_bwd_rows<CH, NC, 1>(b, blocks, s);
+        }
+        return launch_bwd_rows<CH, NC, PIX>(b, blocks, s);
+    };
+    return gradient_channels < CH ? run(std::integral_constant<int, CH - 1>{}) : run(std::integral_constant<int, CH>{});
 }
 
 template <int CH, bool GEOM>
 int launch_bwd(const gs3d_render_bwd_args& b, unsigned blocks, int c0, hipStream_t s) {
     constexpr int PIX = PixFor<CH, true>::value;
-    if constexpr (PIX > 1) {
-        if (blocks < kSmallGrid) return launch_bwd_pix<CH, GEOM, 1>(b, blocks, c0, s);
+    const dim3 grid(blocks), block(kTilePixels / PIX);
+    if constexpr (GEOM) {
+        if (b.abs_centers) {
+            hipLaunchKernelGGL((render_bwd_kernel<CH, true, PIX, true>), grid, block, 0, s, b, c0);
+            return launch_status("gs3d_render_bwd");
+        }
     }
-    return launch_bwd_pix<CH, GEOM, PIX>(b, blocks, c0, s);
+    hipLaunchKernelGGL((render_bwd_kernel<CH, false, PIX, GEOM>), grid, block, 0, s, b, c0);
+    return launch_status("gs3d_render_bwd");
 }
 
 inline int check_render_args(const gs3d_render_args& a) {
@@ -1359,10 +1861,10 @@ extern "C" int gs3d_render_bwd(const gs3d_render_bwd_args* args, void* stream) {
     // Geometry launch over the first window (channels beyond it enter its
     // alpha gradient from global memory), then the feature gradients of the
     // further windows that hold channels with a destination.
-    if (D <= 4) status = launch_bwd<4, true>(b, blocks, 0, s);
-    else if (D <= 8) status = launch_bwd<8, true>(b, blocks, 0, s);
-    else if (D <= 16) status = launch_bwd<16, true>(b, blocks, 0, s);
-    else if (D <= 36) status = launch_bwd<36, true>(b, blocks, 0, s);
+    if (D <= 4) status = launch_bwd_rows<4>(b, blocks, Dg, s);
+    else if (D <= 8) status = launch_bwd_rows<8>(b, blocks, Dg, s);
+    else if (D <= 16) status = launch_bwd_rows<16>(b, blocks, Dg, s);
+    else if (D <= 36) status = launch_bwd_rows<36>(b, blocks, Dg, s);
     else status = launch_bwd<kGeomWindow, true>(b, blocks, 0, s);
     if (status != GS3D_OK || (!b.grad_features && !b.grad_extra)) return status;
     for (int c0 = kGeomWindow; c0 < Dg; c0 += kWindow) {

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import oracle
+from oracle_pipeline import check_gradient
 from dsl_splat_amd.gs3d import render as grender
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +67,53 @@ def test_forward_at_extreme_opacities(width, height, channels):
     np.testing.assert_array_equal(_np(out.stacked()), image)
     assert contributors.max() > 64  # more than one chunk
 
+
+def _backward(width, height, ranges, ids, centers, conics, feats, up, tail=True):
+    """Kernel gradients, the oracle's and their bounds.  Without the constant
+    alpha channel the oracle, which always blends one, gets a zero upstream
+    gradient for it."""
+    out = grender.render_views(ranges, ids, centers, conics, feats, width, height, one_tail=tail)
+    record, grad_features, _ = grender.backward_views(ranges, ids, centers, conics, feats, out.transmittance,
+                                                      out.contributors, up, width, height, absgrad=True,
+                                                      one_tail=tail)
+    up = _np(up) if tail else np.concatenate([_np(up), np.zeros(up.shape[:-1] + (1,), np.float32)], -1)
+    args = (width, height, _np(ranges), _np(ids), _np(centers), _np(conics), _np(feats), _np(out.transmittance),
+            _np(out.contributors), up)
+    rec = _np(record)
+    return (dict(centers=rec[..., 0:2], conics=rec[..., 2:6], abs=rec[..., 6:8], features=_np(grad_features)),
+            oracle.render_bwd(*args, absgrad=True), oracle.render_bwd_bound(*args))
+
+
+# Gradients of every compiled width of the backward, with and without the
+# constant channel, at one and two pixels per lane, through lists whose
+# Gaussians mostly miss the tile: groups of four end anywhere in a batch.
+@pytest.mark.parametrize("width,height,channels,tail", [
+    (75, 43, 1, True), (75, 43, 3, True), (75, 43, 4, False), (75, 43, 7, True), (75, 43, 8, False),
+    (75, 43, 13, True), (75, 43, 16, False), (75, 43, 34, True), (75, 43, 36, False),
+    (1300, 1300, 3, True), (1300, 1300, 4, False), (1300, 1300, 6, True)])
+def test_backward_in_groups(width, height, channels, tail):
+    print("backward in groups", width, height, channels, tail, flush=True)
+    centers, conics, feats, g = _scene(width, height, 400, channels, extreme=False)
+    ids, ranges = _lists(400, width, height, 150, g)
+    up = torch.randn((1, height, width, channels + tail), generator=g).to(DEV)
+    got, ref, bound = _backward(width, height, ranges, ids, centers, conics, feats, up, tail)
+    for name in got:
+        check_gradient(name, got[name], ref[name], bound[name])
+        assert np.abs(got[name]).max() > 0
+
+
+def test_backward_at_extreme_opacities():
+    width, height = 75, 43
+    centers, conics, feats, g = _scene(width, height, 400, 3, extreme=True)
+    # Opacities near the end of the range overflow or not by the order of the
+    # products; NaN and infinite ones do not depend on it.
+    o = conics[..., 3]
+    conics[..., 3] = torch.where((o > 1e30) & (o < float("inf")), torch.full_like(o, 2.0), o)
+    ids, ranges = _lists(400, width, height, 150, g)
+    up = torch.randn((1, height, width, 4), generator=g).to(DEV)
+    got, ref, bound = _backward(width, height, ranges, ids, centers, conics, feats, up)
+    for name in got:
+        finite = np.isfinite(ref[name])
+        np.testing.assert_array_equal(np.isfinite(got[name]), finite, err_msg=name)
+        check_gradient(name, got[name][finite], ref[name][finite],
+                       np.broadcast_to(bound[name], ref[name].shape)[finite])
