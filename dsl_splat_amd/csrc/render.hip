@@ -199,6 +199,15 @@ GS3D_DEV float clamp_exponent(float x) {
     return x;
 }
 
+// A workgroup barrier behind which every LDS operation before it is done.
+// The wait is spelled out: at the head of a loop the compiler leaves it out
+// (it relies on LDS operations of a workgroup running in order, which an
+// atomic that is still on its way from another SIMD does not).
+GS3D_DEV void block_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
 // Lane masks of the whole wavefront as scalars, and a select by one.  Written
 // out as the three-operand form: consecutive two-operand selects on vcc issue
 // six times slower than others on this part (23 against 4.5 cycles in a loop
@@ -635,7 +644,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
         // A barrier that tells whether any wavefront has a live pixel.
         auto any_alive = [&]() {
             if (lane == 0) s_live[wave] = alive();
-            __syncthreads();
+            block_barrier();
             int v = 0;
 #pragma unroll
             for (int w = 0; w < TileWaves<PIX>::count; ++w) v |= s_live[w];
@@ -660,7 +669,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                 }
                 if (begin + B < last) next_id = a.ids[min(begin + B + e, last - 1)];
             }
-            __syncthreads();
+            block_barrier();
             const int cnt = min(B, last - begin);
             bool live = alive();
             for (int c0 = 0; c0 < cnt && live; c0 += 64) {
@@ -744,15 +753,14 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                 };
                 if (strange_color) {
                     at_use(std::false_type{});
-                } else if constexpr ((STATS && (RB > 2 || CH > 4)) || (CH > 16 && CH <= 36)) {
+                } else if constexpr ((STATS && (RB > 2 || CH > 4)) || CH > 16) {
                     // Loads at use: the pipelined form's extra registers would
                     // cost occupancy -- with statistics beyond two requests (their
                     // pixel values take 4 * PIX registers or more) or four
                     // channels (up to both, the pipelined form fits 80 VGPRs),
-                    // and for 36
-                    // channels a third wavefront per SIMD (148 VGPRs against 190
-                    // with the next Gaussian's vector prefetched: 0.83 -> 0.72
-                    // ms on the 32-feature workload).
+                    // and beyond 16 channels a wavefront per SIMD (36 channels:
+                    // 0.83 -> 0.72 ms on the 32-feature workload; 64: 1078 -> 921
+                    // us at 62 channels, 300K Gaussians, 1280x960).
                     at_use(std::true_type{});
                 } else {
                     // Unrolled by two: the next Gaussian is loaded into the other
@@ -787,7 +795,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
         }
         if constexpr (STATS) {
             // The last batch, when the loop ran to the end of the list.
-            __syncthreads();
+            block_barrier();
             flush();
         }
         if constexpr (LISTS != 0) {
@@ -859,7 +867,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
             const int tile = a.redo_list[1 + item];
             if ((unsigned)tile >= (unsigned)tiles) continue;  // uniform: one value per workgroup
             blend(tile_info(a, tile));
-            __syncthreads();
+            block_barrier();
         }
     } else {
         blend(tile_info(a));
@@ -1004,11 +1012,11 @@ GS3D_DEV float upstream_at(const gs3d_render_bwd_args& b, int64_t pix, int gc, i
 // share the LDS that resident workgroups leave.
 template <int CH>
 struct RowsBatch {
-    static constexpr int size = CH <= 8 ? 128 : CH <= 16 ? 256 : 64;
+    static constexpr int size = CH <= 8 ? 128 : CH <= 16 ? 256 : CH <= 20 ? 128 : 64;
 };
 
 template <int CH, int NC, bool ABS, int PIX>
-__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 5 : CH <= 16 ? 4 : 3))) void render_bwd_rows_kernel(gs3d_render_bwd_args b) {
+__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 5 : CH <= 20 ? 4 : CH <= 36 ? 3 : 2))) void render_bwd_rows_kernel(gs3d_render_bwd_args b) {
     constexpr int NT = kTilePixels / PIX;
     constexpr int B = RowsBatch<CH>::size;
     constexpr int FB = ABS ? 8 : 6;
@@ -1093,9 +1101,9 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
         my_max = max(my_max, last_contributor[k]);
     }
     const bool all_finite = lanes(!finite) == 0;
-    __syncthreads();
+    block_barrier();
     if (my_max > 0) atomicMax(&s_max_last, my_max);
-    __syncthreads();
+    block_barrier();
     const int max_last = min(s_max_last, t.last - t.first);
     // The gradient entries this lane adds for its row's Gaussian, one per
     // atomic instruction: an entry of Gaussian g lies at base + g * step.
@@ -1144,7 +1152,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
     // for the next batch loaded while the current one is traversed.
     int32_t next_id = max_last > 0 ? a.ids[t.first + max(max_last - 1 - (int)threadIdx.x, 0)] : 0;
     for (int top = max_last; top > 0; top -= B) {
-        __syncthreads();
+        block_barrier();
         if (threadIdx.x < B) {
             const int e = threadIdx.x;
             const int p = top - 1 - e;
@@ -1155,7 +1163,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
             }
             if (top > B) next_id = a.ids[t.first + max(p - B, 0)];
         }
-        __syncthreads();
+        block_barrier();
         const int cnt = min(B, top);
         // Up to four blended Gaussians: values [pixel][slot], and their batch
         // slots, a byte each.
@@ -1164,72 +1172,72 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
         int used = 0;
         // The gradients of the Gaussians in the slots.
         auto finish = [&]() {
-                            // Row q of lanes: Gaussian q of the four, [pixel][row pair].
-            #pragma unroll
-                            for (int k = 0; k < PIX; ++k) exchange_rows(aT[k], h[k]);
-                            const int j = (slots >> (8 * q)) & 255;
-                            const float4 con = s_g[j].con;
-                            const float2 xy = s_g[j].xy;
-                            const int32_t id = s_id[j];
-                            float dx[PIX], dy[4];
-            #pragma unroll
-                            for (int k = 0; k < PIX; ++k) dx[k] = xy.x - fx[k];
-            #pragma unroll
-                            for (int r = 0; r < 4; ++r) dy[r] = (xy.y - (fy - (float)(2 * q))) - (float)(2 * r);
-                            float v[V];
-                            // Moments over the lane's pixels: per column k the sums of h
-                            // and h dy, per row pair P_r = sum_k h.
-                            float A[PIX], H[PIX], P[4], yy = 0.0f;
-            #pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                P[r] = PIX == 2 ? h[0][r] + h[PIX - 1][r] : h[0][r];
-                                const float py = P[r] * dy[r];
-                                yy = r ? __builtin_fmaf(py, dy[r], yy) : py * dy[r];
-                            }
-            #pragma unroll
-                            for (int k = 0; k < PIX; ++k) {
-                                A[k] = (h[k][0] + h[k][1]) + (h[k][2] + h[k][3]);
-                                H[k] = h[k][0] * dy[0];
-            #pragma unroll
-                                for (int r = 1; r < 4; ++r) H[k] = __builtin_fmaf(h[k][r], dy[r], H[k]);
-                            }
-                            const float mass = PIX == 2 ? A[0] + A[PIX - 1] : A[0];
-                            // The centre gradient from the moments about the middle of
-                            // the lane's pixels (column offsets of 1/2, rows of 1 and 3):
-                            // a dx + b dy may cancel, and is taken there to one rounding.
-                            const float mx = PIX == 2 ? 0.5f * (A[0] - A[PIX - 1]) : 0.0f;
-                            const float my = __builtin_fmaf(3.0f, P[0] - P[3], P[1] - P[2]);
-                            const float dxm = PIX == 2 ? dx[0] - 0.5f : dx[0], dym = dy[0] - 3.0f;
-                            const float ux = dot2_accurate(con.x, dxm, con.y, dym);
-                            const float uy = dot2_accurate(con.z, dym, con.y, dxm);
-                            v[0] = __builtin_fmaf(ux, mass, con.y * my);
-                            v[1] = __builtin_fmaf(uy, mass, con.z * my);
-                            if constexpr (PIX == 2) {
-                                v[0] = __builtin_fmaf(con.x, mx, v[0]);
-                                v[1] = __builtin_fmaf(con.y, mx, v[1]);
-                            }
-                            v[2] = (A[0] * dx[0]) * dx[0];
-                            v[3] = H[0] * dx[0];
-                            if constexpr (PIX == 2) {
-                                v[2] = __builtin_fmaf(A[PIX - 1] * dx[PIX - 1], dx[PIX - 1], v[2]);
-                                v[3] = __builtin_fmaf(H[PIX - 1], dx[PIX - 1], v[3]);
-                            }
-                            v[4] = yy;
-                            v[5] = mass;
-                            if constexpr (ABS) {
-                                v[6] = v[7] = 0.0f;
-            #pragma unroll
-                                for (int r = 0; r < 4; ++r) {
-                                    const float bdy = con.y * dy[r], cdy = con.z * dy[r];
-            #pragma unroll
-                                    for (int k = 0; k < PIX; ++k) {
-                                        const float px = __builtin_fmaf(con.x, dx[k], bdy), py = __builtin_fmaf(con.y, dx[k], cdy);
-                                        v[6] = __builtin_fmaf(__builtin_fabsf(h[k][r]), __builtin_fabsf(px), v[6]);
-                                        v[7] = __builtin_fmaf(__builtin_fabsf(h[k][r]), __builtin_fabsf(py), v[7]);
-                                    }
-                                }
-                            }
-                            // A pixel that did not blend the Gaussian has weight zero; a
+            // Row q of lanes: Gaussian q of the four, [pixel][row pair].
+#pragma unroll
+            for (int k = 0; k < PIX; ++k) exchange_rows(aT[k], h[k]);
+            const int j = (slots >> (8 * q)) & 255;
+            const float4 con = s_g[j].con;
+            const float2 xy = s_g[j].xy;
+            const int32_t id = s_id[j];
+            float dx[PIX], dy[4];
+#pragma unroll
+            for (int k = 0; k < PIX; ++k) dx[k] = xy.x - fx[k];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dy[r] = (xy.y - (fy - (float)(2 * q))) - (float)(2 * r);
+            float v[V];
+            // Moments over the lane's pixels: per column k the sums of h
+            // and h dy, per row pair P_r = sum_k h.
+            float A[PIX], H[PIX], P[4], yy = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                P[r] = PIX == 2 ? h[0][r] + h[PIX - 1][r] : h[0][r];
+                const float py = P[r] * dy[r];
+                yy = r ? __builtin_fmaf(py, dy[r], yy) : py * dy[r];
+            }
+#pragma unroll
+            for (int k = 0; k < PIX; ++k) {
+                A[k] = (h[k][0] + h[k][1]) + (h[k][2] + h[k][3]);
+                H[k] = h[k][0] * dy[0];
+#pragma unroll
+                for (int r = 1; r < 4; ++r) H[k] = __builtin_fmaf(h[k][r], dy[r], H[k]);
+            }
+            const float mass = PIX == 2 ? A[0] + A[PIX - 1] : A[0];
+            // The centre gradient from the moments about the middle of
+            // the lane's pixels (column offsets of 1/2, rows of 1 and 3):
+            // a dx + b dy may cancel, and is taken there to one rounding.
+            const float mx = PIX == 2 ? 0.5f * (A[0] - A[PIX - 1]) : 0.0f;
+            const float my = __builtin_fmaf(3.0f, P[0] - P[3], P[1] - P[2]);
+            const float dxm = PIX == 2 ? dx[0] - 0.5f : dx[0], dym = dy[0] - 3.0f;
+            const float ux = dot2_accurate(con.x, dxm, con.y, dym);
+            const float uy = dot2_accurate(con.z, dym, con.y, dxm);
+            v[0] = __builtin_fmaf(ux, mass, con.y * my);
+            v[1] = __builtin_fmaf(uy, mass, con.z * my);
+            if constexpr (PIX == 2) {
+                v[0] = __builtin_fmaf(con.x, mx, v[0]);
+                v[1] = __builtin_fmaf(con.y, mx, v[1]);
+            }
+            v[2] = (A[0] * dx[0]) * dx[0];
+            v[3] = H[0] * dx[0];
+            if constexpr (PIX == 2) {
+                v[2] = __builtin_fmaf(A[PIX - 1] * dx[PIX - 1], dx[PIX - 1], v[2]);
+                v[3] = __builtin_fmaf(H[PIX - 1], dx[PIX - 1], v[3]);
+            }
+            v[4] = yy;
+            v[5] = mass;
+            if constexpr (ABS) {
+                v[6] = v[7] = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float bdy = con.y * dy[r], cdy = con.z * dy[r];
+#pragma unroll
+                    for (int k = 0; k < PIX; ++k) {
+                        const float px = __builtin_fmaf(con.x, dx[k], bdy), py = __builtin_fmaf(con.y, dx[k], cdy);
+                        v[6] = __builtin_fmaf(__builtin_fabsf(h[k][r]), __builtin_fabsf(px), v[6]);
+                        v[7] = __builtin_fmaf(__builtin_fabsf(h[k][r]), __builtin_fabsf(py), v[7]);
+                    }
+                }
+            }
+            // A pixel that did not blend the Gaussian has weight zero; a
             // non-finite gradient there must not reach it.
             // The widest vectors' gradients do not fit the registers together:
             // four channels of all pixels at a time.
@@ -1246,7 +1254,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
 #pragma unroll
                     for (int c = 0; c < CG; c += 4)
                         *reinterpret_cast<float4*>(u + c) =
-                            *reinterpret_cast<const float4*>(s_grad[wave][i][lane & 15].c + c0 + c);
+            *reinterpret_cast<const float4*>(s_grad[wave][i][lane & 15].c + c0 + c);
                     const float w = aT[i % PIX][i / PIX];
                     if (all_finite) {
 #pragma unroll
@@ -1261,20 +1269,20 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                     if (c0 + c < NC) v[FB + (c0 + c < NC ? c0 + c : 0)] = sum[c];
             }
             sum_rows_packed<V>(v);
-            #pragma unroll
-                            for (int i = 0; i < ATOMICS; ++i) {
-                                float total = v[16 * i];
-            #pragma unroll
-                                for (int m = 1; m < 4; ++m)
-                                    if (16 * i + 4 * m < V) total = ((lane & 3) == m) ? v[16 * i + 4 * m] : total;
-                                total *= dst[i].times_opacity ? dst[i].scale * con.w : dst[i].scale;
-                                // One 32 x 32 -> 64-bit multiply-add for the address (ids
-                                // are non-negative, strides below 2^31).
-                                if (dst[i].base && q < used)
-                                    atomicAdd(dst[i].base + (uint64_t)(uint32_t)id * dst[i].step, total);
-                            }
-                            used = 0;
-                            slots = 0;
+#pragma unroll
+            for (int i = 0; i < ATOMICS; ++i) {
+                float total = v[16 * i];
+#pragma unroll
+                for (int m = 1; m < 4; ++m)
+                    if (16 * i + 4 * m < V) total = ((lane & 3) == m) ? v[16 * i + 4 * m] : total;
+                total *= dst[i].times_opacity ? dst[i].scale * con.w : dst[i].scale;
+                // One 32 x 32 -> 64-bit multiply-add for the address (ids
+                // are non-negative, strides below 2^31).
+                if (dst[i].base && q < used)
+                    atomicAdd(dst[i].base + (uint64_t)(uint32_t)id * dst[i].step, total);
+            }
+            used = 0;
+            slots = 0;
         };
         for (int c0 = 0; c0 < cnt; c0 += 64) {
             // This wavefront's Gaussians of the next 64 that lie before its
@@ -1466,9 +1474,9 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
         }
         my_max = max(my_max, last_contributor[k]);
     }
-    __syncthreads();
+    block_barrier();
     if (my_max > 0) atomicMax(&s_max_last, my_max);
-    __syncthreads();
+    block_barrier();
     const int max_last = min(s_max_last, t.last - t.first);
     // Gradient entry this lane adds after the wavefront sums (see
     // wave_sum_rows): entry k of Gaussian g lives at dst_base + g * dst_step.
@@ -1515,7 +1523,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
     static_assert(B <= NT, "one staged Gaussian per thread and batch");
     int32_t next_id = max_last > 0 ? a.ids[t.first + max(max_last - 1 - (int)threadIdx.x, 0)] : 0;
     for (int top = max_last; top > 0; top -= B) {
-        __syncthreads();
+        block_barrier();
         if (threadIdx.x < B) {
             const int e = threadIdx.x;
             const int p = top - 1 - e;
@@ -1529,7 +1537,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
             }
             if (top > B) next_id = a.ids[t.first + max(p - B, 0)];
         }
-        __syncthreads();
+        block_barrier();
         const int cnt = min(B, top);
         for (int c0b = 0; c0b < cnt; c0b += 64) {
           // This wavefront's Gaussians of the next 64 that lie before its
@@ -1708,13 +1716,21 @@ int launch_fwd(const gs3d_render_args& a, const gs3d_render_stats_args* st, unsi
     return launch_fwd_pix<CH, PIX>(a, st, counts, blocks, c0, s);
 }
 
-// One forward window of `width` channels starting at c0.
+// One forward window of `width` channels starting at c0.  Every slot of a
+// kernel's width costs a multiply-add per accepted pixel and 4 bytes of LDS
+// per staged Gaussian, so the widths follow what is blended: colours with a
+// depth (4, 8), descriptors of 16, 32 and 40 channels with one or two more (20,
+// 36, 44).  300K Gaussians at 1280x960, forward and backward: 18 channels in
+// 36 slots 343 + 689, in 20 220 + 410 us; 42 in 64 and 56 slots 1024 + 1353, in
+// 44 467 + 1075 us.
 inline int launch_fwd_window(const gs3d_render_args& a, const gs3d_render_stats_args* st, unsigned long long* counts,
                              unsigned blocks, int c0, int width, hipStream_t s) {
     if (width <= 4) return launch_fwd<4>(a, st, counts, blocks, c0, s);
     if (width <= 8) return launch_fwd<8>(a, st, counts, blocks, c0, s);
     if (width <= 16) return launch_fwd<16>(a, st, counts, blocks, c0, s);
+    if (width <= 20) return launch_fwd<20>(a, st, counts, blocks, c0, s);
     if (width <= 36) return launch_fwd<36>(a, st, counts, blocks, c0, s);
+    if (width <= 44) return launch_fwd<44>(a, st, counts, blocks, c0, s);
     return launch_fwd<kWindow>(a, st, counts, blocks, c0, s);
 }
 
@@ -1864,7 +1880,9 @@ extern "C" int gs3d_render_bwd(const gs3d_render_bwd_args* args, void* stream) {
     if (D <= 4) status = launch_bwd_rows<4>(b, blocks, Dg, s);
     else if (D <= 8) status = launch_bwd_rows<8>(b, blocks, Dg, s);
     else if (D <= 16) status = launch_bwd_rows<16>(b, blocks, Dg, s);
+    else if (D <= 20) status = launch_bwd_rows<20>(b, blocks, Dg, s);
     else if (D <= 36) status = launch_bwd_rows<36>(b, blocks, Dg, s);
+    else if (D <= 44) status = launch_bwd_rows<44>(b, blocks, Dg, s);
     else status = launch_bwd<kGeomWindow, true>(b, blocks, 0, s);
     if (status != GS3D_OK || (!b.grad_features && !b.grad_extra)) return status;
     for (int c0 = kGeomWindow; c0 < Dg; c0 += kWindow) {

@@ -51,10 +51,11 @@ def _scene(width, height, n, channels, extreme):
     return centers.to(DEV), conics.to(DEV), torch.randn((n, channels), generator=g).to(DEV), g
 
 
-# Fewer than 4096 tiles: one pixel per lane; more: two.  Channels: every
+# Fewer than 6144 tiles: one pixel per lane; more: two.  Channels: every
 # compiled width of the forward.
-@pytest.mark.parametrize("width,height,channels", [(75, 43, 3), (75, 43, 7), (75, 43, 13), (75, 43, 34),
-                                                   (1030, 1027, 3), (1030, 1027, 6)])
+@pytest.mark.parametrize("width,height,channels", [(75, 43, 3), (75, 43, 7), (75, 43, 13), (75, 43, 18),
+                                                   (75, 43, 34), (75, 43, 41), (75, 43, 60),
+                                                   (1300, 1300, 3), (1300, 1300, 6)])
 def test_forward_at_extreme_opacities(width, height, channels):
     print("forward extreme opacities", width, height, channels, flush=True)
     centers, conics, feats, g = _scene(width, height, 400, channels, extreme=True)
@@ -89,7 +90,8 @@ def _backward(width, height, ranges, ids, centers, conics, feats, up, tail=True)
 # Gaussians mostly miss the tile: groups of four end anywhere in a batch.
 @pytest.mark.parametrize("width,height,channels,tail", [
     (75, 43, 1, True), (75, 43, 3, True), (75, 43, 4, False), (75, 43, 7, True), (75, 43, 8, False),
-    (75, 43, 13, True), (75, 43, 16, False), (75, 43, 34, True), (75, 43, 36, False),
+    (75, 43, 13, True), (75, 43, 16, False), (75, 43, 18, True), (75, 43, 20, False), (75, 43, 34, True),
+    (75, 43, 41, True), (75, 43, 44, False), (75, 43, 36, False),
     (1300, 1300, 3, True), (1300, 1300, 4, False), (1300, 1300, 6, True)])
 def test_backward_in_groups(width, height, channels, tail):
     print("backward in groups", width, height, channels, tail, flush=True)
