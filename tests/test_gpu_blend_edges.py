@@ -119,3 +119,25 @@ def test_backward_at_extreme_opacities():
         np.testing.assert_array_equal(np.isfinite(got[name]), finite, err_msg=name)
         check_gradient(name, got[name][finite], ref[name][finite],
                        np.broadcast_to(bound[name], ref[name].shape)[finite])
+
+
+@pytest.mark.parametrize("width,height", [(75, 43), (1300, 1300)])
+def test_non_finite_channels_and_gradients(width, height):
+    # One and two pixels per lane: a non-finite channel or upstream gradient
+    # reaches what blended it and nothing else.
+    centers, conics, feats, g = _scene(width, height, 400, 3, extreme=False)
+    ids, ranges = _lists(400, width, height, 150, g)
+    feats[11, 0] = float("nan")
+    feats[12, 1] = float("inf")
+    out = grender.render_views(ranges, ids, centers, conics, feats, width, height)
+    image, _, _ = oracle.render_fwd(width, height, _np(ranges), _np(ids), _np(centers), _np(conics), _np(feats))
+    np.testing.assert_array_equal(_np(out.stacked()), image)
+    up = torch.randn((1, height, width, 4), generator=g).to(DEV)
+    up[0, height // 2, width // 3, 0] = float("nan")
+    up[0, height // 3, width // 2, 1] = float("-inf")
+    got, ref, bound = _backward(width, height, ranges, ids, centers, conics, feats, up)
+    for name in got:
+        finite = np.isfinite(ref[name])
+        np.testing.assert_array_equal(np.isfinite(got[name]), finite, err_msg=name)
+        check_gradient(name, got[name][finite], ref[name][finite],
+                       np.broadcast_to(bound[name], ref[name].shape)[finite])
