@@ -185,8 +185,8 @@ GS3D_DEV void wave_sum_rows(const float (&v)[V], float (&out)[(V + 3) / 4]) {
     constexpr int R = (V + 3) / 4;
     float w[W];
     if constexpr (V <= 16) {
-        // Up to 16 entries (the 4- and 8-channel blend VJPs, the statistics
-        // observer): the swaps as in-place instructions on copies the
+        // Up to 16 entries (the statistics observer, the blend VJP's narrow
+        // feature windows): the swaps as in-place instructions on copies the
         // wavefront sum owns, so both operands are consumed and no register
         // is copied out first.  The compiler cannot see the swap inside the
         // asm, so the wait states it needs after a VALU write of its operands
