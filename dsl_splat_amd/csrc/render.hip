@@ -307,10 +307,18 @@ struct alignas(16) StagedRec {
     float f[CH];
 };
 
-// Strip-mask bit of a Gaussian whose opacity (kStrange) is not finite or one
-// of whose staged channels (kStrangeColor) is not: the blend loops take their
-// cases apart.
-constexpr uint32_t kStrange = 1u << 31, kStrangeColor = 1u << 30;
+// Strip-mask bit of a Gaussian whose opacity (kStrange) is not finite, one of
+// whose staged channels (kStrangeColor) is not, or one of whose conic entries
+// (kSharp) is beyond kMomentConic: the blend loops take their cases apart.
+constexpr uint32_t kStrange = 1u << 31, kStrangeColor = 1u << 30, kSharp = 1u << 29;
+
+// Largest conic entry whose centre gradient the backward takes from moments.
+// They are formed about the middle of a lane's pixels, blended or not: beside
+// a pixel within a standard deviation of the centre that loses about sqrt(a)
+// * 2^-24 of the gradient, and overflows for entries near the end of the
+// range.  Projection dilates covariances by 0.3 (entries below 3.34); sharper
+// conics come from geometry made by hand and are summed pixel by pixel.
+constexpr float kMomentConic = 4.0f;
 
 // Stage one Gaussian's centre, conic, cutoff, strip mask and the channels
 // [c0, c0 + CH) of its channel vector (zero beyond D').
@@ -365,6 +373,8 @@ GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32
     }
     if (top >= 0x7F800000u) mask |= kStrangeColor;
     if (limit == __builtin_inff()) mask |= kStrange;
+    if (!(sel_max(sel_max(__builtin_fabsf(con.x), __builtin_fabsf(con.y)), __builtin_fabsf(con.z)) <= kMomentConic))
+        mask |= kSharp;
     s_mask[slot] = mask;
 }
 
@@ -1170,6 +1180,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
         float aT[PIX][4], h[PIX][4];
         uint32_t slots = 0;
         int used = 0;
+        bool sharp = false;  // one of the batch's Gaussians so far is kSharp
         // The gradients of the Gaussians in the slots.
         auto finish = [&]() {
             // Row q of lanes: Gaussian q of the four, [pixel][row pair].
@@ -1216,14 +1227,6 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                 v[0] = __builtin_fmaf(con.x, mx, v[0]);
                 v[1] = __builtin_fmaf(con.y, mx, v[1]);
             }
-            v[2] = (A[0] * dx[0]) * dx[0];
-            v[3] = H[0] * dx[0];
-            if constexpr (PIX == 2) {
-                v[2] = __builtin_fmaf(A[PIX - 1] * dx[PIX - 1], dx[PIX - 1], v[2]);
-                v[3] = __builtin_fmaf(H[PIX - 1], dx[PIX - 1], v[3]);
-            }
-            v[4] = yy;
-            v[5] = mass;
             if constexpr (ABS) {
                 v[6] = v[7] = 0.0f;
 #pragma unroll
@@ -1237,6 +1240,14 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                     }
                 }
             }
+            v[2] = (A[0] * dx[0]) * dx[0];
+            v[3] = H[0] * dx[0];
+            if constexpr (PIX == 2) {
+                v[2] = __builtin_fmaf(A[PIX - 1] * dx[PIX - 1], dx[PIX - 1], v[2]);
+                v[3] = __builtin_fmaf(H[PIX - 1], dx[PIX - 1], v[3]);
+            }
+            v[4] = yy;
+            v[5] = mass;
             // A pixel that did not blend the Gaussian has weight zero; a
             // non-finite gradient there must not reach it.
             // The widest vectors' gradients do not fit the registers together:
@@ -1268,6 +1279,29 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                 for (int c = 0; c < CG; ++c)
                     if (c0 + c < NC) v[FB + (c0 + c < NC ? c0 + c : 0)] = sum[c];
             }
+            if (sharp) {
+                // Their centre gradients again, pixel by pixel: a pixel that did
+                // not blend the Gaussian (h = 0) adds nothing, whatever its
+                // product with the conic.
+                v[0] = v[1] = 0.0f;
+                if constexpr (ABS) v[6] = v[7] = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+#pragma unroll
+                    for (int k = 0; k < PIX; ++k) {
+                        const float hp = h[k][r];
+                        const float px = __builtin_fmaf(con.x, dx[k], con.y * dy[r]);
+                        const float py = __builtin_fmaf(con.z, dy[r], con.y * dx[k]);
+                        const float tx = hp != 0.0f ? hp * px : 0.0f, ty = hp != 0.0f ? hp * py : 0.0f;
+                        v[0] += tx;
+                        v[1] += ty;
+                        if constexpr (ABS) {
+                            v[6] += __builtin_fabsf(tx);
+                            v[7] += __builtin_fabsf(ty);
+                        }
+                    }
+                }
+            }
             sum_rows_packed<V>(v);
 #pragma unroll
             for (int i = 0; i < ATOMICS; ++i) {
@@ -1291,6 +1325,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
             const uint32_t flags = s_mask[min(slot0, B - 1)];
             uint64_t todo = lanes(slot0 < cnt && top - 1 - slot0 < wave_last && ((flags >> wave) & 1u));
             const bool strange = (lanes((flags & kStrange) != 0) & todo) != 0;
+            sharp |= (lanes((flags & kSharp) != 0) & todo) != 0;
             while (todo) {
                 // One Gaussian undone from this lane's pixels: its weight and h.
                 const int j = c0 + __builtin_ctzll(todo);

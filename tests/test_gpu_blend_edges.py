@@ -121,6 +121,42 @@ def test_backward_at_extreme_opacities():
                        np.broadcast_to(bound[name], ref[name].shape)[finite])
 
 
+# Conics far sharper than projection's (its 0.3 px dilation keeps entries below
+# 3.4), to the end of the range, on or just beside pixel centres: one pixel of
+# a lane blends the Gaussian, its neighbours' products with the conic overflow
+# or are many orders larger than the blending pixel's.
+@pytest.mark.parametrize("width,height,channels", [(75, 43, 3), (75, 43, 13), (75, 43, 18), (75, 43, 34),
+                                                   (75, 43, 41), (75, 43, 50), (1300, 1300, 3)])
+def test_backward_at_extreme_conics(width, height, channels):
+    print("backward extreme conics", width, height, channels, flush=True)
+    centers, conics, feats, g = _scene(width, height, 400, channels, extreme=False)
+    centers, conics = centers.cpu(), conics.cpu()
+    m = 200
+    scale = 10.0 ** (torch.arange(m) % 20 * 2.0)           # 1 to 1e38
+    a, c = (scale * (1.0 + torch.rand(m, generator=g)) for _ in range(2))
+    conics[0, :m, 0], conics[0, :m, 2] = a, c
+    conics[0, :m, 1] = (torch.rand(m, generator=g) * 2 - 1) * a.sqrt() * c.sqrt() * 0.9
+    conics[0, :m, 3] = 0.5
+    # Within one standard deviation of a pixel of the first rows and columns,
+    # where small offsets are representable; a third exactly on it.
+    centers[0, :m] = torch.randint(0, 3, (m, 2), generator=g) + \
+        (torch.rand((m, 2), generator=g) - 0.5) / scale.sqrt()[:, None]
+    centers[0, :m:3] = centers[0, :m:3].round()
+    centers, conics = centers.to(DEV), conics.to(DEV)
+    ids, ranges = _lists(400, width, height, 150, g)
+    up = torch.randn((1, height, width, channels + 1), generator=g).to(DEV)
+    got, ref, bound = _backward(width, height, ranges, ids, centers, conics, feats, up)
+    for name in got:
+        finite = np.isfinite(ref[name])
+        np.testing.assert_array_equal(np.isfinite(got[name]), finite, err_msg=name)
+        # The absolute tolerance is of the magnitude of 1: entries of sharp
+        # Gaussians' centres reach 1e19 and only rtol and the bound apply.
+        check_gradient(name, got[name][finite], ref[name][finite],
+                       np.broadcast_to(bound[name], ref[name].shape)[finite])
+    blended = np.abs(ref["features"][:m]).max(-1) > 0
+    assert blended.reshape(-1, 20).any(0).all()            # every scale reaches a pixel
+
+
 @pytest.mark.parametrize("width,height", [(75, 43), (1300, 1300)])
 def test_non_finite_channels_and_gradients(width, height):
     # One and two pixels per lane: a non-finite channel or upstream gradient
