@@ -303,13 +303,14 @@ struct alignas(16) StagedRec {
     float4 con;
     float2 xy;
     float limit;  // exponent_limit
-    int entry;    // list position, 1-based
+    int entry;    // list position, 1-based (forward)
     float f[CH];
 };
 
-// Strip-mask bit of a Gaussian whose opacity (kStrange) is not finite, one of
-// whose staged channels (kStrangeColor) is not, or one of whose conic entries
-// (kSharp) is beyond kMomentConic: the blend loops take their cases apart.
+// Strip-mask bit of a Gaussian whose opacity (kStrange) is not finite (in the
+// grouped backward: or beyond kHugeOpacity), one of whose staged channels
+// (kStrangeColor) is not finite, or one of whose conic entries (kSharp) is
+// beyond kMomentConic: the blend loops take their cases apart.
 constexpr uint32_t kStrange = 1u << 31, kStrangeColor = 1u << 30, kSharp = 1u << 29;
 
 // Largest conic entry whose centre gradient the backward takes from moments.
@@ -320,9 +321,15 @@ constexpr uint32_t kStrange = 1u << 31, kStrangeColor = 1u << 30, kSharp = 1u <<
 // conics come from geometry made by hand and are summed pixel by pixel.
 constexpr float kMomentConic = 4.0f;
 
+// Beyond this opacity e^power of a blended pixel may be so small that its
+// product with the pixel's gradient falls below the normal range; the grouped
+// backward keeps it times kHugeScale there, and stages the opacity over it.
+constexpr float kHugeOpacity = 0x1p64f, kHugeScale = 0x1p64f;
+
 // Stage one Gaussian's centre, conic, cutoff, strip mask and the channels
-// [c0, c0 + CH) of its channel vector (zero beyond D').
-template <int CH, int PIX, bool LAUNDER = false>
+// [c0, c0 + CH) of its channel vector (zero beyond D').  SCALED: the record's
+// entry holds 1, or 1 / kHugeScale where the opacity is staged times that.
+template <int CH, int PIX, bool LAUNDER = false, bool SCALED = false>
 GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32_t g, int slot, int entry, int c0,
                              StagedRec<CH>* s_g, uint32_t* s_mask) {
     const int view = t.view;
@@ -353,7 +360,14 @@ GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32
     rec.xy = xy;
     const float limit = exponent_limit(con.w);
     rec.limit = limit;
-    rec.entry = entry;
+    const bool huge = con.w > kHugeOpacity && con.w < __builtin_inff();
+    if constexpr (SCALED) {
+        const float scale = huge ? 1.0f / kHugeScale : 1.0f;
+        rec.con.w = con.w * scale;
+        rec.entry = __float_as_int(scale);
+    } else {
+        rec.entry = entry;
+    }
     int x0 = t.x0, y0 = t.y0;
     if constexpr (LAUNDER) {
         // The tile origin passes through an opaque scalar move, so that the
@@ -372,7 +386,7 @@ GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32
         top = max(top, __float_as_uint(v[c]) & 0x7FFFFFFFu);
     }
     if (top >= 0x7F800000u) mask |= kStrangeColor;
-    if (limit == __builtin_inff()) mask |= kStrange;
+    if (limit == __builtin_inff() || (SCALED && huge)) mask |= kStrange;
     if (!(sel_max(sel_max(__builtin_fabsf(con.x), __builtin_fabsf(con.y)), __builtin_fabsf(con.z)) <= kMomentConic))
         mask |= kSharp;
     s_mask[slot] = mask;
@@ -1121,13 +1135,13 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
         float* base;
         uint32_t step;  // row strides below 2^31 (checked on the host)
         float scale;
-        bool times_opacity;
+        bool times_opacity, is_opacity;
     } dst[ATOMICS];
 #pragma unroll
     for (int i = 0; i < ATOMICS; ++i) {
         const int k = 4 * (4 * i + (lane & 3)) + row_bank_value(lane);
         const int64_t row0 = (int64_t)t.view * a.n;
-        Destination d = {nullptr, 0, 1.0f, k < FB && k != 5};
+        Destination d = {nullptr, 0, 1.0f, k < FB && k != 5, k == 5};
         if (k < 2 || k == 3) d.scale = -1.0f;
         if (k == 2 || k == 4) d.scale = -0.5f;
         if (k >= V) {
@@ -1169,7 +1183,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
             const int32_t g = next_id;
             if (p >= 0) {
                 s_id[e] = g;
-                stage_gaussian<CH, PIX, true>(a, t, g, e, p + 1, 0, s_g, s_mask);
+                stage_gaussian<CH, PIX, true, true>(a, t, g, e, 0, 0, s_g, s_mask);
             }
             if (top > B) next_id = a.ids[t.first + max(p - B, 0)];
         }
@@ -1189,6 +1203,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
             const int j = (slots >> (8 * q)) & 255;
             const float4 con = s_g[j].con;
             const float2 xy = s_g[j].xy;
+            const float unscale = __int_as_float(s_g[j].entry);
             const int32_t id = s_id[j];
             float dx[PIX], dy[4];
 #pragma unroll
@@ -1309,7 +1324,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
 #pragma unroll
                 for (int m = 1; m < 4; ++m)
                     if (16 * i + 4 * m < V) total = ((lane & 3) == m) ? v[16 * i + 4 * m] : total;
-                total *= dst[i].times_opacity ? dst[i].scale * con.w : dst[i].scale;
+                if (i == 0) total *= dst[0].times_opacity ? dst[0].scale * con.w : dst[0].is_opacity ? unscale : 1.0f;
                 // One 32 x 32 -> 64-bit multiply-add for the address (ids
                 // are non-negative, strides below 2^31).
                 if (dst[i].base && q < used)
@@ -1346,7 +1361,10 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                 float G[PIX], alpha[PIX], weight[PIX], hv[PIX];
                 if (strange) {
 #pragma unroll
-                    for (int k = 0; k < PIX; ++k) G[k] = blend_exp(-x[k]);
+                    for (int k = 0; k < PIX; ++k) {
+                        G[k] = blend_exp(-x[k]);
+                        if (__int_as_float(g.entry) != 1.0f) G[k] *= kHugeScale;
+                    }
                 } else {
 #pragma unroll
                     for (int k = 0; k < PIX; ++k) G[k] = blend_exp_neg(x[k]);

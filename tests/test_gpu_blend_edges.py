@@ -121,6 +121,28 @@ def test_backward_at_extreme_opacities():
                        np.broadcast_to(bound[name], ref[name].shape)[finite])
 
 
+# Finite opacities to the end of the range with small upstream gradients: no
+# product overflows, but e^power is as small as 1e-38 and its product with the
+# upstream gradient alone would lose its bits below the normal range.
+@pytest.mark.parametrize("width,height,channels", [(75, 43, 3), (75, 43, 13), (75, 43, 18), (75, 43, 34),
+                                                   (75, 43, 50), (1300, 1300, 3)])
+def test_backward_at_huge_opacities(width, height, channels):
+    print("backward huge opacities", width, height, channels, flush=True)
+    centers, conics, feats, g = _scene(width, height, 400, channels, extreme=False)
+    o = conics[0, :, 3].cpu()
+    o[::2] = 10.0 ** (torch.arange(200) % 39).float()
+    conics[0, :, 3] = o.to(DEV)
+    ids, ranges = _lists(400, width, height, 150, g)
+    up = torch.randn((1, height, width, channels + 1), generator=g).to(DEV) * 1e-6
+    got, ref, bound = _backward(width, height, ranges, ids, centers, conics, feats, up)
+    for name in got:
+        # The absolute tolerance scaled by the upstream gradients.
+        finite = np.isfinite(ref[name])
+        np.testing.assert_array_equal(np.isfinite(got[name]), finite, err_msg=name)
+        check_gradient(name, got[name][finite], ref[name][finite],
+                       np.broadcast_to(bound[name], ref[name].shape)[finite], atol=1e-11)
+
+
 # Conics far sharper than projection's (its 0.3 px dilation keeps entries below
 # 3.4), to the end of the range, on or just beside pixel centres: one pixel of
 # a lane blends the Gaussian, its neighbours' products with the conic overflow
