@@ -1285,37 +1285,54 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
             }
             v[4] = yy;
             v[5] = mass;
-            // A pixel that did not blend the Gaussian has weight zero; a
-            // non-finite gradient there must not reach it.
-            // The widest vectors' gradients do not fit the registers together:
-            // four channels of all pixels at a time.
-            constexpr int CG = NC > 16 ? 4 : NC;
+            // The colour sums, four pixels and four channels at a time, so that
+            // no more gradients hold registers.  Beyond 8 channels the next
+            // ones are on their way from LDS while the ones before are added
+            // (42 channels of a 256x256 frame 272 -> 257 us); below, that would
+            // spill, or cost a wavefront per SIMD (8 channels 240 -> 258 us at
+            // 1237x822).  Choosing by all_finite per load had made a block of
+            // each, waiting for LDS one by one: 36 channels of a 256x256 frame
+            // 322 -> 232 us, of 1M Gaussians 4x1080p 6440 -> 5080 us.  A pixel
+            // that did not blend the Gaussian has weight zero; a non-finite
+            // gradient there must not reach it.
+            auto colors = [&](auto finite) {
+                constexpr bool FINITE = decltype(finite)::value;
+                constexpr int STEPS = (NC + 3) / 4 * PIX;
+                constexpr bool AHEAD = CH > 8;
+                float4 u[2][4];
+                auto load = [&](int step) {
 #pragma unroll
-            for (int c0 = 0; c0 < NC; c0 += CG) {
-                if constexpr (CG < NC) asm volatile("" ::: "memory");
-                float sum[CG];
+                    for (int i = 0; i < 4; ++i)
+                        u[step & 1][i] = *reinterpret_cast<const float4*>(
+                            s_grad[wave][4 * (step % PIX) + i][lane & 15].c + 4 * (step / PIX));
+                };
+                if constexpr (AHEAD) load(0);
 #pragma unroll
-                for (int c = 0; c < CG; ++c) sum[c] = 0.0f;
+                for (int step = 0; step < STEPS; ++step) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (!AHEAD) load(step);
+                    else if (step + 1 < STEPS) load(step + 1);
+                    float sum[4];
 #pragma unroll
-                for (int i = 0; i < 4 * PIX; ++i) {
-                    alignas(16) float u[(CG + 3) / 4 * 4];
+                    for (int c = 0; c < 4; ++c) {
+                        const int cc = 4 * (step / PIX) + c;
+                        if (cc >= NC) continue;
+                        sum[c] = step % PIX ? v[FB + (cc < NC ? cc : 0)] : 0.0f;
 #pragma unroll
-                    for (int c = 0; c < CG; c += 4)
-                        *reinterpret_cast<float4*>(u + c) =
-            *reinterpret_cast<const float4*>(s_grad[wave][i][lane & 15].c + c0 + c);
-                    const float w = aT[i % PIX][i / PIX];
-                    if (all_finite) {
-#pragma unroll
-                        for (int c = 0; c < CG; ++c) sum[c] = __builtin_fmaf(w, u[c], sum[c]);
-                    } else {
-#pragma unroll
-                        for (int c = 0; c < CG; ++c) sum[c] += w != 0.0f ? w * u[c] : 0.0f;
+                        for (int i = 0; i < 4; ++i) {
+                            const int p = 4 * (step % PIX) + i;
+                            const float w = aT[p % PIX][p / PIX];
+                            const float4 g4 = u[step & 1][i];
+                            const float g1 = c == 0 ? g4.x : c == 1 ? g4.y : c == 2 ? g4.z : g4.w;
+                            sum[c] = FINITE ? __builtin_fmaf(w, g1, sum[c]) : sum[c] + (w != 0.0f ? w * g1 : 0.0f);
+                        }
+                        v[FB + (cc < NC ? cc : 0)] = sum[c];
                     }
                 }
-#pragma unroll
-                for (int c = 0; c < CG; ++c)
-                    if (c0 + c < NC) v[FB + (c0 + c < NC ? c0 + c : 0)] = sum[c];
-            }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            if (all_finite) colors(std::true_type{});
+            else colors(std::false_type{});
             if (sharp) {
                 // Their centre gradients again, pixel by pixel: a pixel that did
                 // not blend the Gaussian (h = 0) adds nothing, whatever its
