@@ -327,9 +327,10 @@ constexpr float kMomentConic = 4.0f;
 constexpr float kHugeOpacity = 0x1p64f, kHugeScale = 0x1p64f;
 
 // Stage one Gaussian's centre, conic, cutoff, strip mask and the channels
-// [c0, c0 + CH) of its channel vector (zero beyond D').  SCALED: the record's
-// entry holds 1, or 1 / kHugeScale where the opacity is staged times that.
-template <int CH, int PIX, bool LAUNDER = false, bool SCALED = false>
+// [c0, c0 + CH) of its channel vector (zero beyond D').  GROUPED, for the
+// grouped backward: sharp conics are marked, and the record's entry holds 1, or
+// 1 / kHugeScale where the opacity is staged times that.
+template <int CH, int PIX, bool LAUNDER = false, bool GROUPED = false>
 GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32_t g, int slot, int entry, int c0,
                              StagedRec<CH>* s_g, uint32_t* s_mask) {
     const int view = t.view;
@@ -360,8 +361,8 @@ GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32
     rec.xy = xy;
     const float limit = exponent_limit(con.w);
     rec.limit = limit;
-    const bool huge = con.w > kHugeOpacity && con.w < __builtin_inff();
-    if constexpr (SCALED) {
+    const bool huge = GROUPED && con.w > kHugeOpacity && con.w < __builtin_inff();
+    if constexpr (GROUPED) {
         const float scale = huge ? 1.0f / kHugeScale : 1.0f;
         rec.con.w = con.w * scale;
         rec.entry = __float_as_int(scale);
@@ -386,9 +387,11 @@ GS3D_DEV void stage_gaussian(const gs3d_render_args& a, const TileInfo& t, int32
         top = max(top, __float_as_uint(v[c]) & 0x7FFFFFFFu);
     }
     if (top >= 0x7F800000u) mask |= kStrangeColor;
-    if (limit == __builtin_inff() || (SCALED && huge)) mask |= kStrange;
-    if (!(sel_max(sel_max(__builtin_fabsf(con.x), __builtin_fabsf(con.y)), __builtin_fabsf(con.z)) <= kMomentConic))
-        mask |= kSharp;
+    if (limit == __builtin_inff() || huge) mask |= kStrange;
+    if constexpr (GROUPED) {
+        if (!(sel_max(sel_max(__builtin_fabsf(con.x), __builtin_fabsf(con.y)), __builtin_fabsf(con.z)) <= kMomentConic))
+            mask |= kSharp;
+    }
     s_mask[slot] = mask;
 }
 
@@ -1863,9 +1866,11 @@ int launch_bwd_rows(const gs3d_render_bwd_args& b, unsigned blocks, int gradient
     return gradient_channels < CH ? run(std::integral_constant<int, CH - 1>{}) : run(std::integral_constant<int, CH>{});
 }
 
-template <int CH, bool GEOM>
+template <int CH, bool GEOM, int PIX = PixFor<CH, true>::value>
 int launch_bwd(const gs3d_render_bwd_args& b, unsigned blocks, int c0, hipStream_t s) {
-    constexpr int PIX = PixFor<CH, true>::value;
+    if constexpr (PIX > 1) {
+        if (blocks < kSmallGrid) return launch_bwd<CH, GEOM, 1>(b, blocks, c0, s);
+    }
     const dim3 grid(blocks), block(kTilePixels / PIX);
     if constexpr (GEOM) {
         if (b.abs_centers) {
