@@ -540,7 +540,10 @@ GS3D_DEV void observe_statistics(const gs3d_render_stats_args& st, int dst_r, fl
 
 // Up to 4 channels the kernel is held to 80 VGPRs (6 wavefronts per SIMD
 // instead of 5: 1.180 -> 1.130 ms on RGB), up to 8 to 96, up to 36 to 168 (3
-// wavefronts).  Lane masks, weights of zero and the exponential from adds
+// wavefronts), beyond to 256 (2: 64 slots left to themselves took 284 to 302
+// registers and one wavefront, 60 channels at 1237x822 893 against 549 us, with
+// two statistics 1075 against 643).  Wide kernels spill a few tens of registers
+// at these bounds, most of them with statistics.  Lane masks, weights of zero and the exponential from adds
 // (see the file comment): 3M Gaussians, 4 x 1920x1080, 1005 -> 790 us; 500K
 // at 1280x720 169 -> 138 us; 34 channels at 1600x1200 688 -> 596 us.
 //
@@ -561,7 +564,7 @@ GS3D_DEV void observe_statistics(const gs3d_render_stats_args& st, int dst_r, fl
 // capped launch.  Only the instantiations that use them carry the stop
 // tracking and the loop.
 template <int CH, int PIX, int MODE, int RB = 1, int KINDS = -1, int LISTS = 0>
-__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 6 : CH <= 8 ? 5 : CH <= 36 ? 3 : 1))) void render_fwd_kernel(gs3d_render_args a, gs3d_render_stats_args st, int c0, unsigned long long* counts) {
+__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 6 : CH <= 8 ? 5 : CH <= 36 ? 3 : 2))) void render_fwd_kernel(gs3d_render_args a, gs3d_render_stats_args st, int c0, unsigned long long* counts) {
     constexpr bool STATS = MODE == 1, COUNTS = MODE == 2;
     constexpr int NT = kTilePixels / PIX;
     constexpr int B = Batch<CH>::size;
