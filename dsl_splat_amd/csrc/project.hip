@@ -1080,13 +1080,16 @@ __global__ __launch_bounds__(kShRowBlock) void sh_rows_bwd_kernel(gs3d_project_b
 }
 
 // The standalone SH evaluation and its VJP, one thread per row of `rows`
-// coefficients, of which the degree needs E floats.  Both are bound by HBM:
-// rows that start on 16 bytes (VEC) are read as float4, and the VJP's gradient
-// rows of exactly RF floats (zero beyond E) leave through the wavefront's LDS
-// slice in coalesced copies, as a row of 48 floats comes in where all of it
-// is needed.  RF 0: per-lane accesses of any row length and alignment.  1M
-// rows of 16 coefficients at degree 3: VJP 634 -> 69 us (a row indexed at run
-// time had put the gradients in scratch memory), forward 67 -> 46 us.
+// coefficients, of which the degree needs E floats.  Both are bound by HBM.
+// The forward reads and writes its rows per lane, with plain stores: a lane's
+// three floats are a part of a line, which the L2 merges (streamed, 4M rows at
+// degree 0 took 26 against 18 us and 1M of degree 3 33 against 31; float4
+// loads changed nothing).  In the VJP rows that start on 16 bytes (VEC) are
+// read as float4, and gradient rows of exactly RF floats (zero beyond E) leave
+// through the wavefront's LDS slice in coalesced copies, as a row of 48 floats
+// comes in where all of it is needed.  RF 0: per-lane accesses of any row
+// length and alignment.  1M rows of 16 coefficients at degree 3: VJP 625 -> 65
+// us (a row indexed at run time had put the gradients in scratch memory).
 template <int E, bool VEC>
 GS3D_DEV void load_sh_row(const float* src, float (&coef)[E]) {
     if constexpr (VEC) {
@@ -1104,7 +1107,7 @@ GS3D_DEV void load_sh_row(const float* src, float (&coef)[E]) {
     }
 }
 
-template <int DEG, bool VEC>
+template <int DEG>
 __global__ __launch_bounds__(256) void sh_fwd_kernel(const float* __restrict__ coefficients, int rows,
                                                      const float* __restrict__ dirs,
                                                      const int32_t* __restrict__ radii, int n,
@@ -1113,13 +1116,13 @@ __global__ __launch_bounds__(256) void sh_fwd_kernel(const float* __restrict__ c
     if (i >= n) return;
     constexpr int KC = (DEG + 1) * (DEG + 1);
     float coef[3 * KC];
-    load_sh_row<3 * KC, VEC>(coefficients + i * rows * 3, coef);
+    for (int e = 0; e < 3 * KC; ++e) coef[e] = coefficients[i * rows * 3 + e];
     const float dir[3] = {dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2]};
     const bool vis = radii ? radii[i] > 0 : true;
     float color[3], raw[3];
     sh_eval<DEG>(coef, dir, vis, color, raw);
     for (int k = 0; k < 3; ++k) {
-        st_stream(colors + 3 * i + k, color[k]);
+        colors[3 * i + k] = color[k];
         if (active) active[3 * i + k] = (vis && raw[k] >= 0.0f) ? 1 : 0;
     }
 }
@@ -1192,14 +1195,8 @@ __global__ __launch_bounds__(kShBlock) void sh_bwd_kernel(const float* __restric
 template <int DEG>
 int launch_sh_fwd(const float* coefficients, int rows, const float* directions, const int32_t* radii, int n,
                   float* colors, uint8_t* active, hipStream_t s) {
-    // Whole float4s from the row's start: the last one may pass the degree's
-    // coefficients, never the row.
-    const bool vec = (reinterpret_cast<uintptr_t>(coefficients) & 15) == 0 && (rows * 3) % 4 == 0;
     const dim3 grid(blocks_for(n, 256)), block(256);
-    if (vec)
-        hipLaunchKernelGGL((sh_fwd_kernel<DEG, true>), grid, block, 0, s, coefficients, rows, directions, radii, n, colors, active);
-    else
-        hipLaunchKernelGGL((sh_fwd_kernel<DEG, false>), grid, block, 0, s, coefficients, rows, directions, radii, n, colors, active);
+    hipLaunchKernelGGL((sh_fwd_kernel<DEG>), grid, block, 0, s, coefficients, rows, directions, radii, n, colors, active);
     return launch_status("gs3d_sh_fwd");
 }
 
