@@ -1156,8 +1156,12 @@ __global__ __launch_bounds__(kShBlock) void sh_bwd_kernel(const float* __restric
     if constexpr (RF == E) {
         static_assert(RF == 0 || PITCH == RF + 1, "rows_to_lds' pitch");
         rows_to_lds<RF>(stage, coefficients + g0 * RF, rows_here);
+        const float* const row_in = stage + min(lane, rows_here - 1) * PITCH;
 #pragma unroll
-        for (int e = 0; e < E; ++e) coef[e] = row_lds[e];
+        for (int e = 0; e < E; ++e) coef[e] = row_in[e];
+        // Read by every lane before gradient rows take their place.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     } else {
         load_sh_row<E, RF != 0>(coefficients + i * rows * 3, coef);
     }
@@ -1208,7 +1212,9 @@ int launch_sh_bwd(const float* coefficients, int rows, const float* directions, 
         ((reinterpret_cast<uintptr_t>(coefficients) | reinterpret_cast<uintptr_t>(grad_coefficients)) & 15) == 0;
     const dim3 grid(blocks_for(n, kShBlock)), block(kShBlock);
     // Rows of 16 coefficients (any degree of a trainer's schedule) and of the
-    // 4 that degree 1 needs; other rows are rare.
+    // 4 that degree 1 needs; rows of other lengths, among them the 1 and 9 of
+    // degrees 0 and 2 by themselves, are written per lane (1M rows 5 and 50 us
+    // where staged rows of 4 take 21 and of 16 65).
     if (aligned && rows == 16)
         hipLaunchKernelGGL((sh_bwd_kernel<DEG, 48>), grid, block, 0, s, coefficients, rows, directions, radii, active, upstream, n, grad_coefficients, grad_directions);
     else if (DEG == 1 && aligned && rows == 4)
