@@ -1762,14 +1762,30 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
 // small frame still spreads over the SIMDs.  Each tile's list is walked
 // serially; at two pixels per lane a few thousand tiles make little more than
 // one full set of resident wavefronts (6 per SIMD, 6144 on the chip), and the
-// longest lists set the time.  Forward and backward at one against two pixels
-// per lane: three 801x601 views (5814 tiles) 281 + 474 against 323 + 569 us;
-// 1920x1080 with very large Gaussians (8160 tiles) 312 + 1169 against 289 +
-// 733 us; two 1920x1080 views (16320 tiles) 389 + 800 against 367 + 672 us.
+// longest lists set the time.  Forward at one against two pixels per lane:
+// 300K Gaussians at 1152x960 (4320 tiles) 115 against 132 us, at 1600x1200
+// (7500 tiles) 152 against 152.
+//
+// The backward adds a Gaussian's gradients once per wavefront, so there one
+// pixel per lane means twice the atomics, and these are the bound where large
+// Gaussians are many.  From kSmallGridBwd tiles it is taken only if the
+// frame's lists are known to hold few entries per Gaussian (and view).  One
+// against two pixels per lane, 4 channels: 1152x960 with 13 entries per Gaussian
+// 196 against 222 us, with 38 147 against 166, with 103 420 against 253;
+// 1440x1040 with 19 220 against 254, with 52 171 against 168, with 146 567
+// against 315.
 #ifndef GS3D_SMALL_GRID
 #define GS3D_SMALL_GRID 6144
 #endif
-constexpr unsigned kSmallGrid = GS3D_SMALL_GRID;
+constexpr unsigned kSmallGrid = GS3D_SMALL_GRID, kSmallGridBwd = 4096;
+constexpr int64_t kEntriesPerGaussian = 40;
+
+// ids_count: the lists' entries in all, or negative if not known.
+inline bool small_grid_bwd(const gs3d_render_args& a, unsigned blocks, int64_t ids_count) {
+    if (blocks < kSmallGridBwd) return true;
+    return blocks < kSmallGrid && ids_count >= 0 && ids_count <= kEntriesPerGaussian * a.n * a.views;
+}
+
 // Workgroups of a redo launch (gs3d_render_args.redo_pass).
 constexpr unsigned kRedoGrid = 512;
 
@@ -1857,12 +1873,12 @@ int launch_bwd_rows(const gs3d_render_bwd_args& b, unsigned blocks, hipStream_t 
 
 // All gradients of a vector of at most 16 channels.
 template <int CH>
-int launch_bwd_rows(const gs3d_render_bwd_args& b, unsigned blocks, int gradient_channels, hipStream_t s) {
+int launch_bwd_rows(const gs3d_render_bwd_args& b, unsigned blocks, bool small, int gradient_channels, hipStream_t s) {
     constexpr int PIX = PixFor<CH, true>::value;
     auto run = [&](auto nc) {
         constexpr int NC = decltype(nc)::value;
         if constexpr (PIX > 1) {
-            if (blocks < kSmallGrid) return launch_bwd_rows<CH, NC, 1>(b, blocks, s);
+            if (small) return launch_bwd_rows<CH, NC, 1>(b, blocks, s);
         }
         return launch_bwd_rows<CH, NC, PIX>(b, blocks, s);
     };
@@ -1870,9 +1886,9 @@ int launch_bwd_rows(const gs3d_render_bwd_args& b, unsigned blocks, int gradient
 }
 
 template <int CH, bool GEOM, int PIX = PixFor<CH, true>::value>
-int launch_bwd(const gs3d_render_bwd_args& b, unsigned blocks, int c0, hipStream_t s) {
+int launch_bwd(const gs3d_render_bwd_args& b, unsigned blocks, bool small, int c0, hipStream_t s) {
     if constexpr (PIX > 1) {
-        if (blocks < kSmallGrid) return launch_bwd<CH, GEOM, 1>(b, blocks, c0, s);
+        if (small) return launch_bwd<CH, GEOM, 1>(b, blocks, small, c0, s);
     }
     const dim3 grid(blocks), block(kTilePixels / PIX);
     if constexpr (GEOM) {
@@ -1965,6 +1981,10 @@ extern "C" int gs3d_render_fwd_stats(const gs3d_render_args* args, const gs3d_re
 }
 
 extern "C" int gs3d_render_bwd(const gs3d_render_bwd_args* args, void* stream) {
+    return gs3d_render_bwd_lists(args, -1, stream);
+}
+
+extern "C" int gs3d_render_bwd_lists(const gs3d_render_bwd_args* args, int64_t ids_count, void* stream) {
     if (!args) return GS3D_ERR_ARGUMENT;
     const gs3d_render_bwd_args& b = *args;
     const gs3d_render_args& a = b.fwd;
@@ -1986,25 +2006,26 @@ extern "C" int gs3d_render_bwd(const gs3d_render_bwd_args* args, void* stream) {
     const int D = a.feat_channels + a.extra_channels + (a.one_tail ? 1 : 0);
     const int Dg = D - (a.one_tail ? 1 : 0);
     const unsigned blocks = render_blocks(a);
+    const bool small = small_grid_bwd(a, blocks, ids_count);
     hipStream_t s = as_stream(stream);
     // Geometry launch over the first window (channels beyond it enter its
     // alpha gradient from global memory), then the feature gradients of the
     // further windows that hold channels with a destination.
-    if (D <= 4) status = launch_bwd_rows<4>(b, blocks, Dg, s);
-    else if (D <= 8) status = launch_bwd_rows<8>(b, blocks, Dg, s);
-    else if (D <= 16) status = launch_bwd_rows<16>(b, blocks, Dg, s);
-    else if (D <= 20) status = launch_bwd_rows<20>(b, blocks, Dg, s);
-    else if (D <= 36) status = launch_bwd_rows<36>(b, blocks, Dg, s);
-    else if (D <= 44) status = launch_bwd_rows<44>(b, blocks, Dg, s);
-    else status = launch_bwd<kGeomWindow, true>(b, blocks, 0, s);
+    if (D <= 4) status = launch_bwd_rows<4>(b, blocks, small, Dg, s);
+    else if (D <= 8) status = launch_bwd_rows<8>(b, blocks, small, Dg, s);
+    else if (D <= 16) status = launch_bwd_rows<16>(b, blocks, small, Dg, s);
+    else if (D <= 20) status = launch_bwd_rows<20>(b, blocks, small, Dg, s);
+    else if (D <= 36) status = launch_bwd_rows<36>(b, blocks, small, Dg, s);
+    else if (D <= 44) status = launch_bwd_rows<44>(b, blocks, small, Dg, s);
+    else status = launch_bwd<kGeomWindow, true>(b, blocks, small, 0, s);
     if (status != GS3D_OK || (!b.grad_features && !b.grad_extra)) return status;
     for (int c0 = kGeomWindow; c0 < Dg; c0 += kWindow) {
         const int width = min(kWindow, D - c0);
-        if (width <= 4) status = launch_bwd<4, false>(b, blocks, c0, s);
-        else if (width <= 8) status = launch_bwd<8, false>(b, blocks, c0, s);
-        else if (width <= 16) status = launch_bwd<16, false>(b, blocks, c0, s);
-        else if (width <= 36) status = launch_bwd<36, false>(b, blocks, c0, s);
-        else status = launch_bwd<kWindow, false>(b, blocks, c0, s);
+        if (width <= 4) status = launch_bwd<4, false>(b, blocks, small, c0, s);
+        else if (width <= 8) status = launch_bwd<8, false>(b, blocks, small, c0, s);
+        else if (width <= 16) status = launch_bwd<16, false>(b, blocks, small, c0, s);
+        else if (width <= 36) status = launch_bwd<36, false>(b, blocks, small, c0, s);
+        else status = launch_bwd<kWindow, false>(b, blocks, small, c0, s);
         if (status != GS3D_OK) return status;
     }
     return GS3D_OK;

@@ -226,7 +226,7 @@ def backward_views(ranges: Tensor, ids: Tensor, centers: Tensor, conics: Tensor,
         b.grad_extra = native.ptr(grad_extra)
         b.grad_extra_stride = extra.shape[-1]
         b.grad_extra_view_stride = n * extra.shape[-1] if extra.ndim == 3 else 0
-    native.call("gs3d_render_bwd", ctypes.byref(b), native.stream(device))
+    native.call("gs3d_render_bwd_lists", ctypes.byref(b), ids.numel(), native.stream(device))
     return record, grad_features, grad_extra
 
 

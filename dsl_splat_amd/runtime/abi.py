@@ -306,4 +306,5 @@ FUNCTIONS = {
     "gs3d_render_pair_counts": (ctypes.c_int, [ctypes.POINTER(RenderArgs), _P, _P]),
     "gs3d_render_fwd_stats": (ctypes.c_int, [ctypes.POINTER(RenderArgs), ctypes.POINTER(RenderStatsArgs), _P]),
     "gs3d_render_bwd": (ctypes.c_int, [ctypes.POINTER(RenderBwdArgs), _P]),
+    "gs3d_render_bwd_lists": (ctypes.c_int, [ctypes.POINTER(RenderBwdArgs), _I64, _P]),
 }

@@ -532,6 +532,11 @@ typedef struct gs3d_render_bwd_args {
 
 int gs3d_render_bwd(const gs3d_render_bwd_args* args, void* stream);
 
+/* gs3d_render_bwd for a caller that knows how many entries the tile lists hold
+ * in all (ids_count; negative: not known, as gs3d_render_bwd).  Same results;
+ * the launch shape of mid-size grids follows the entries per Gaussian. */
+int gs3d_render_bwd_lists(const gs3d_render_bwd_args* args, int64_t ids_count, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -122,6 +122,7 @@ def test_argument_errors_are_reported_without_launching():
     bwd.grad_centers = bwd.grad_conics = ctypes.c_void_p(256)
     bwd.grad_centers_stride, bwd.grad_conics_stride = 1 << 31, 4
     assert lib.gs3d_render_bwd(ctypes.byref(bwd), None) == abi.GS3D_ERR_ARGUMENT
+    assert lib.gs3d_render_bwd_lists(ctypes.byref(bwd), 100, None) == abi.GS3D_ERR_ARGUMENT
     # Zero-size work is a no-op.
     assert lib.gs3d_pair_tiles(None, 0, None, 0, None) == abi.GS3D_OK
     args = abi.BinArgs()

@@ -104,6 +104,21 @@ def test_backward_in_groups(width, height, channels, tail):
         assert np.abs(got[name]).max() > 0
 
 
+# Grids of 4096 to 6143 tiles: two pixels per lane beyond 40 list entries per
+# Gaussian, one up to them, and 8 channels in a further window after 56.
+@pytest.mark.parametrize("n,channels", [(400, 3), (17_000, 3), (400, 58), (17_000, 58)])
+def test_backward_of_mid_size_grids(n, channels):
+    width, height = 1152, 960
+    print("backward mid-size grid", n, channels, flush=True)
+    centers, conics, feats, g = _scene(width, height, n, channels, extreme=False)
+    ids, ranges = _lists(n, width, height, 150, g)
+    assert 4096 <= len(ranges) < 6144 and (ids.numel() > 40 * n) == (n == 400)
+    up = torch.randn((1, height, width, channels + 1), generator=g).to(DEV)
+    got, ref, bound = _backward(width, height, ranges, ids, centers, conics, feats, up)
+    for name in got:
+        check_gradient(name, got[name], ref[name], bound[name])
+
+
 def test_backward_at_extreme_opacities():
     width, height = 75, 43
     centers, conics, feats, g = _scene(width, height, 400, 3, extreme=True)
