@@ -1061,15 +1061,19 @@ GS3D_DEV float upstream_at(const gs3d_render_bwd_args& b, int64_t pix, int gc, i
 // 1280x720 with absolute gradients 304 -> 227 us; 78K at 637x421 with 9
 // channels 238 -> 177 us.  The pixels' gradients for the second half lie in LDS: in registers
 // (24 more) the kernel spilled or lost a wavefront per SIMD.
+//
 // Gaussians staged per batch: the staged channels and the pixels' gradients
-// share the LDS that resident workgroups leave.
+// share the LDS that resident workgroups leave.  9 to 16 channels hold three
+// wavefronts per SIMD with 256 (43 KB); 128 would make it four, 3340 -> 2995 us
+// for 13 channels of 1M Gaussians 4x1080p, and cost frames that have fewer
+// wavefronts than that their staging rounds, 145 -> 158 us at 256x256.
 template <int CH>
 struct RowsBatch {
     static constexpr int size = CH <= 8 ? 128 : CH <= 16 ? 256 : CH <= 20 ? 128 : 64;
 };
 
 template <int CH, int NC, bool ABS, int PIX>
-__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 5 : CH <= 20 ? 4 : CH <= 36 ? 3 : 2))) void render_bwd_rows_kernel(gs3d_render_bwd_args b) {
+__global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 5 : CH <= 8 ? 4 : CH <= 16 ? 3 : CH <= 20 ? 4 : CH <= 36 ? 3 : 2))) void render_bwd_rows_kernel(gs3d_render_bwd_args b) {
     constexpr int NT = kTilePixels / PIX;
     constexpr int B = RowsBatch<CH>::size;
     constexpr int FB = ABS ? 8 : 6;
