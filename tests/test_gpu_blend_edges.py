@@ -10,6 +10,7 @@ import torch
 import oracle
 from oracle_pipeline import check_gradient
 from dsl_splat_amd.gs3d import render as grender
+from test_gpu_stages import assert_two_pixels
 
 pytestmark = pytest.mark.gpu
 
@@ -25,7 +26,10 @@ def _np(t):
 
 def _lists(n, width, height, per_tile, g):
     """Tile lists that are not derived from footprints: each tile lists
-    `per_tile` Gaussians, most of them far outside it."""
+    `per_tile` Gaussians, most of them far outside it.  Frames of 1300x1300
+    stand for the two-pixel kernels."""
+    if (width, height) == (1300, 1300):
+        assert_two_pixels(width, height)
     tiles = ((width + 15) // 16) * ((height + 15) // 16)
     ids = torch.stack([torch.randperm(n, generator=g)[:per_tile] for _ in range(tiles)]).int().flatten()
     first = torch.arange(tiles, dtype=torch.int32) * per_tile
@@ -119,15 +123,17 @@ def test_backward_of_mid_size_grids(n, channels):
         check_gradient(name, got[name], ref[name], bound[name])
 
 
-def test_backward_at_extreme_opacities():
-    width, height = 75, 43
-    centers, conics, feats, g = _scene(width, height, 400, 3, extreme=True)
+@pytest.mark.parametrize("width,height,channels", [(75, 43, 3), (75, 43, 13), (75, 43, 34), (1300, 1300, 3),
+                                                   (1300, 1300, 6)])
+def test_backward_at_extreme_opacities(width, height, channels):
+    print("backward extreme opacities", width, height, channels, flush=True)
+    centers, conics, feats, g = _scene(width, height, 400, channels, extreme=True)
     # Opacities near the end of the range overflow or not by the order of the
     # products; NaN and infinite ones do not depend on it.
     o = conics[..., 3]
     conics[..., 3] = torch.where((o > 1e30) & (o < float("inf")), torch.full_like(o, 2.0), o)
     ids, ranges = _lists(400, width, height, 150, g)
-    up = torch.randn((1, height, width, 4), generator=g).to(DEV)
+    up = torch.randn((1, height, width, channels + 1), generator=g).to(DEV)
     got, ref, bound = _backward(width, height, ranges, ids, centers, conics, feats, up)
     for name in got:
         finite = np.isfinite(ref[name])
@@ -194,20 +200,22 @@ def test_backward_at_extreme_conics(width, height, channels):
     assert blended.reshape(-1, 20).any(0).all()            # every scale reaches a pixel
 
 
-@pytest.mark.parametrize("width,height", [(75, 43), (1300, 1300)])
-def test_non_finite_channels_and_gradients(width, height):
+@pytest.mark.parametrize("width,height,channels", [(75, 43, 3), (75, 43, 7), (75, 43, 13), (75, 43, 18), (75, 43, 34),
+                                                   (75, 43, 41), (75, 43, 60), (1300, 1300, 3), (1300, 1300, 6)])
+def test_non_finite_channels_and_gradients(width, height, channels):
     # One and two pixels per lane: a non-finite channel or upstream gradient
-    # reaches what blended it and nothing else.
-    centers, conics, feats, g = _scene(width, height, 400, 3, extreme=False)
+    # reaches what blended it and nothing else, in every compiled width.
+    print("non-finite", width, height, channels, flush=True)
+    centers, conics, feats, g = _scene(width, height, 400, channels, extreme=False)
     ids, ranges = _lists(400, width, height, 150, g)
     feats[11, 0] = float("nan")
-    feats[12, 1] = float("inf")
+    feats[12, channels - 1] = float("inf")
     out = grender.render_views(ranges, ids, centers, conics, feats, width, height)
     image, _, _ = oracle.render_fwd(width, height, _np(ranges), _np(ids), _np(centers), _np(conics), _np(feats))
     np.testing.assert_array_equal(_np(out.stacked()), image)
-    up = torch.randn((1, height, width, 4), generator=g).to(DEV)
+    up = torch.randn((1, height, width, channels + 1), generator=g).to(DEV)
     up[0, height // 2, width // 3, 0] = float("nan")
-    up[0, height // 3, width // 2, 1] = float("-inf")
+    up[0, height // 3, width // 2, channels - 1] = float("-inf")
     got, ref, bound = _backward(width, height, ranges, ids, centers, conics, feats, up)
     for name in got:
         finite = np.isfinite(ref[name])

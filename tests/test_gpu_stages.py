@@ -8,13 +8,16 @@ rtol 1e-4 / atol 1e-5 of the oracle's or within its stated float32 error
 bound (oracle_pipeline.check_gradient).
 """
 
+import os
+import re
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
 from oracle_pipeline import check_gradient, compare
-from dsl_splat_amd import gs3d, synthetic
+from dsl_splat_amd import build, gs3d, synthetic
 from dsl_splat_amd.gs3d import projection as gproj
 from dsl_splat_amd.gs3d import render as grender
 from dsl_splat_amd.primitives import tiling
@@ -34,25 +37,42 @@ def _say(*args):
     print(*args, flush=True)
 
 
-# Frames of fewer than 4096 tiles (all views) blend at one pixel per lane,
-# larger ones at two: the "wide" scenes (4320 tiles) cover the two-pixel
-# kernels.
+# Frames of fewer tiles (all views) than the blends' GS3D_SMALL_GRID run at one
+# pixel per lane, larger ones at two: the "wide" scenes (6724 and 6400 tiles)
+# cover the two-pixel kernels, and assert_two_pixels that they still do.
 SCENES = {
     "small_rgb": dict(name="small", n=4000, width=128, height=96, seed=1),
     "sh3_4view": dict(name="sh3_1080p_4view", n=6000, width=160, height=96, seed=2),
     "sh3_720p": dict(name="sh3_720p", n=5000, width=200, height=120, seed=3),
-    "wide_rgb": dict(name="small", n=16000, width=1152, height=960, seed=11),
-    "wide_sh3_4view": dict(name="sh3_1080p_4view", n=12000, width=576, height=480, seed=12),
+    "wide_rgb": dict(name="small", n=16000, width=1300, height=1300, seed=11),
+    "wide_sh3_4view": dict(name="sh3_1080p_4view", n=12000, width=640, height=640, seed=12),
     # 4 tile groups and ~1.5M group items: the group sort's 32 digit rows
     # over more than 512 sort tiles take the two-launch digit scan.
     "dense_small": dict(name="small", n=1_500_000, width=256, height=256, seed=21),
 }
 
 
+def _tiles(width, height, views=1):
+    return views * ((width + 15) // 16) * ((height + 15) // 16)
+
+
+def small_grid():
+    """Tiles below which the blends run at one pixel per lane."""
+    with open(os.path.join(build.CSRC, "render.hip")) as f:
+        return int(re.search(r"#define GS3D_SMALL_GRID (\d+)", f.read()).group(1))
+
+
+def assert_two_pixels(width, height, views=1):
+    assert _tiles(width, height, views) >= small_grid(), "this frame no longer runs the two-pixel blends"
+
+
 def _scene(key):
     cfg = dict(SCENES[key])
     name = cfg.pop("name")
-    return synthetic.make_scene(name, **cfg).to(DEV)
+    scene = synthetic.make_scene(name, **cfg).to(DEV)
+    if key.startswith("wide"):
+        assert_two_pixels(scene.width, scene.height, scene.viewmats.shape[0])
+    return scene
 
 
 def _project(scene, sh_degree=None):
@@ -213,12 +233,14 @@ def test_render_forward_bit_exact(key, degree, extra, bg):
     assert ct.max() > 0
 
 
-@pytest.mark.parametrize("n,width,height", [(3000, 136, 100), (12000, 1152, 960)])
+@pytest.mark.parametrize("n,width,height", [(3000, 136, 100), (12000, 1300, 1300)])
 def test_render_culling_edge_cases(n, width, height):
     # Needle-shaped Gaussians at every orientation and opacities straddling
     # the 1/255 threshold: the per-wavefront strip culling must not change a
     # single forward bit or the gradients (one and two pixels per lane).
     _say(f"render culling edge cases {width}x{height}")
+    if width > 1000:
+        assert_two_pixels(width, height)
     scene = synthetic.make_scene("small", n=n, width=width, height=height, seed=5)
     g = torch.Generator().manual_seed(7)
     n = scene.means.shape[0]

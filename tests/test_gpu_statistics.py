@@ -113,12 +113,15 @@ def _stats_against_oracle(scene, feats, st, bins, kinds, pv, nonfinite=False):
 # Request counts of every compiled bucket (1, 2, 4, 8), every combination of
 # kinds of one and two requests (compiled in), at one and two pixels per lane
 # and at 4 and 8 blended channels (4-channel launches of up to two requests
-# take the pipelined traversal; the others load at use).
+# take the pipelined traversal; the others load at use), and every wider kernel
+# (16, 20, 36, 44 and 64 channels).
 @pytest.mark.parametrize("key,channels,kinds", [
     ("small_rgb", 3, (1,)), ("wide_rgb", 3, (1,)), ("wide_rgb", 3, (0,)), ("wide_rgb", 3, (0, 1)),
     ("wide_rgb", 3, (1, 0)), ("wide_rgb", 3, (0, 0)), ("wide_rgb", 3, (1, 1)), ("wide_rgb", 3, (0, 1, 1)),
     ("wide_rgb", 3, (1, 0, 1, 1, 0, 1, 0, 0)), ("wide_rgb", 6, (1,)), ("wide_rgb", 6, (0, 1)),
-    ("small_rgb", 6, (0, 1, 0, 1))])
+    ("wide_rgb", 6, (1, 0, 1, 1, 0, 1, 0, 0)), ("small_rgb", 6, (0, 1, 0, 1)), ("small_rgb", 13, (0, 1)),
+    ("small_rgb", 18, (1,)), ("small_rgb", 31, (0, 1, 1)), ("small_rgb", 41, (1, 0, 1, 1, 0, 1, 0, 0)),
+    ("small_rgb", 55, (0, 1)), ("small_rgb", 60, (1, 0, 1, 1, 0, 1, 0, 0))])
 def test_statistics_request_buckets(key, channels, kinds):
     scene = _scene(key)
     _say(f"statistics buckets {key} D={channels} kinds={kinds}")
