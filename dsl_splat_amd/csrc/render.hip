@@ -211,7 +211,7 @@ GS3D_DEV void block_barrier() {
 
 // Lane masks of the whole wavefront as scalars, and a select by one.  Written
 // out as the three-operand form: consecutive two-operand selects on vcc issue
-// six times slower than others on this part (23 against 4.5 cycles in a loop
+// five times slower than others on this part (23 against 4.5 cycles in a loop
 // of them).
 GS3D_DEV uint64_t lanes(bool v) { return __builtin_amdgcn_ballot_w64(v); }
 GS3D_DEV float select(uint64_t mask, float yes, float no) {
@@ -788,7 +788,8 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
                     // Loads at use: the pipelined form's extra registers would
                     // cost occupancy -- with statistics beyond two requests (their
                     // pixel values take 4 * PIX registers or more) or four
-                    // channels (up to both, the pipelined form fits 80 VGPRs),
+                    // channels (up to both, the pipelined form is held to 80
+                    // VGPRs with up to seven spilled at two pixels per lane),
                     // and beyond 16 channels a wavefront per SIMD (36 channels:
                     // 0.83 -> 0.72 ms on the 32-feature workload; 64: 1078 -> 921
                     // us at 62 channels, 300K Gaussians, 1280x960).
@@ -929,7 +930,7 @@ GS3D_DEV float rest_dot(const gs3d_render_bwd_args& b, int view, int64_t g, floa
 }
 
 // ---------------------------------------------------------------------------
-// Backward, up to 16 channels: four Gaussians at a time
+// Backward, up to 44 channels: four Gaussians at a time
 //
 // The gradients of a Gaussian are sums over pixels that depend on a pixel
 // through two numbers, the blend weight alpha T (colour gradients) and
@@ -1053,16 +1054,6 @@ GS3D_DEV float upstream_at(const gs3d_render_bwd_args& b, int64_t pix, int gc, i
     return has ? u : 0.0f;
 }
 
-// D <= CH channels, of which at most NC have gradients (the constant alpha
-// channel, last, has none).  Bound by vector instructions: at two pixels per
-// lane about 90 per Gaussian undo it from the pixels and 35 are its share of a
-// group's sums; without the atomics the kernel takes 1% less where Gaussians
-// are small and 24% less where some cover thousands of tiles.  3M Gaussians,
-// 4 x 1920x1080: 1640 -> 1455 us (94 VGPRs, five wavefronts per SIMD); 500K at
-// 1280x720 with absolute gradients 304 -> 227 us; 78K at 637x421 with 9
-// channels 238 -> 177 us.  The pixels' gradients for the second half lie in LDS: in registers
-// (24 more) the kernel spilled or lost a wavefront per SIMD.
-//
 // Gaussians staged per batch: the staged channels and the pixels' gradients
 // share the LDS that resident workgroups leave.  9 to 16 channels hold three
 // wavefronts per SIMD with 256 (43 KB); 128 would make it four, 3340 -> 2995 us
@@ -1073,6 +1064,16 @@ struct RowsBatch {
     static constexpr int size = CH <= 8 ? 128 : CH <= 16 ? 256 : CH <= 20 ? 128 : 64;
 };
 
+// D <= CH channels, of which at most NC have gradients (the constant alpha
+// channel, last, has none).  Bound by vector instructions: at two pixels per
+// lane about 90 per Gaussian undo it from the pixels and 35 are its share of a
+// group's sums; without the atomics the kernel takes 1% less where Gaussians
+// are small and 24% less where some cover thousands of tiles.  Against one
+// Gaussian at a time: 1M Gaussians 4x1080p 1615 -> 1345 us (94 VGPRs, five
+// wavefronts per SIMD), with 18 channels 6600 -> 2770, with 36 6910 -> 5080;
+// 400K at 1237x822 283 -> 224, with 9 channels 448 -> 360.  The pixels'
+// gradients for the second half lie in LDS: in registers (24 more) the kernel
+// spilled or lost a wavefront per SIMD.
 template <int CH, int NC, bool ABS, int PIX>
 __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_eu(CH <= 4 ? 5 : CH <= 8 ? 4 : CH <= 16 ? 3 : CH <= 20 ? 4 : CH <= 36 ? 3 : 2))) void render_bwd_rows_kernel(gs3d_render_bwd_args b) {
     constexpr int NT = kTilePixels / PIX;
@@ -1515,8 +1516,8 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
     const TileInfo t = tile_info(a);
     const int D = a.feat_channels + a.extra_channels + (a.one_tail ? 1 : 0);
     const int Dg = D - (a.one_tail ? 1 : 0);
-    // Only the widest geometry window can be followed by further channels.
-    const bool rest = GEOM && CH == kGeomWindow && D > CH;  // wave-uniform
+    static_assert(!GEOM || CH == kGeomWindow, "narrower vectors run the grouped backward");
+    const bool rest = GEOM && D > CH;  // channels beyond the window; wave-uniform
     const int lane = lane_id(), wave = threadIdx.x >> 6;
     // Per pixel: S = sum_c accum_c * grad_c, the colour accumulated behind
     // the current Gaussian dotted with the upstream gradient.  With
@@ -1646,9 +1647,7 @@ __global__ __launch_bounds__(kTilePixels / PIX) __attribute__((amdgpu_waves_per_
             const int32_t g = next_id;
             if (p >= 0) {
                 s_id[e] = g;
-                // Tile origin laundered (see stage_gaussian): 75 instead of
-                // 79 VGPRs, no spill with absolute gradients, 1.7% faster
-                // at 36 channels.
+                // Tile origin laundered (see stage_gaussian).
                 stage_gaussian<CH, PIX, true>(a, t, g, e, p + 1, c0, s_g, s_mask);
             }
             if (top > B) next_id = a.ids[t.first + max(p - B, 0)];
@@ -1849,12 +1848,20 @@ int launch_fwd(const gs3d_render_args& a, const gs3d_render_stats_args* st, unsi
 }
 
 // One forward window of `width` channels starting at c0.  Every slot of a
-// kernel's width costs a multiply-add per accepted pixel and 4 bytes of LDS
-// per staged Gaussian, so the widths follow what is blended: colours with a
-// depth (4, 8), descriptors of 16, 32 and 40 channels with one or two more (20,
-// 36, 44).  300K Gaussians at 1280x960, forward and backward: 18 channels in
-// 36 slots 343 + 689, in 20 220 + 410 us; 42 in 64 and 56 slots 1024 + 1353, in
-// 44 467 + 1075 us.
+// kernel's width costs a multiply-add per accepted pixel, 4 bytes of LDS per
+// staged Gaussian and registers, so the lines lie where a wider kernel holds
+// fewer wavefronts per SIMD: up to 20 slots four (110 registers forward, 128
+// backward), 36 three (168), beyond two.  44 is the line of the grouped
+// backward (59 of 64 KB LDS, 225 registers); the kernels of 64 and 56 slots are
+// what is left.  17 to 20 channels in 36 slots against 20, and 37 to 44 in 64
+// and 56 against 44, forward and backward in us:
+//   300K Gaussians 1280x960   17: 264 + 515, 207 + 320     20: 282 + 516, 230 + 330
+//                             37: 503 + 1255, 434 + 788    44: 525 + 1282, 465 + 826
+//   10K Gaussians 256x256     17: 105 + 234, 88 + 159      44: 145 + 379, 123 + 257
+//   100K, some very large,    17: 414 + 976, 348 + 856     44: 794 + 2143, 716 + 2120
+//   1920x1080
+// What still rides in wider slots: 21 channels 278 + 518, 45 channels 525 + 1290
+// at 1280x960.
 inline int launch_fwd_window(const gs3d_render_args& a, const gs3d_render_stats_args* st, unsigned long long* counts,
                              unsigned blocks, int c0, int width, hipStream_t s) {
     if (width <= 4) return launch_fwd<4>(a, st, counts, blocks, c0, s);
@@ -1876,7 +1883,7 @@ int launch_bwd_rows(const gs3d_render_bwd_args& b, unsigned blocks, hipStream_t 
     return launch_status("gs3d_render_bwd");
 }
 
-// All gradients of a vector of at most 16 channels.
+// All gradients of a vector of at most 44 channels.
 template <int CH>
 int launch_bwd_rows(const gs3d_render_bwd_args& b, unsigned blocks, bool small, int gradient_channels, hipStream_t s) {
     constexpr int PIX = PixFor<CH, true>::value;
