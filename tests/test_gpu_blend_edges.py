@@ -10,6 +10,7 @@ import torch
 import oracle
 from oracle_pipeline import check_gradient
 from dsl_splat_amd.gs3d import render as grender
+from dsl_splat_amd.runtime import native
 from test_gpu_stages import assert_two_pixels
 
 pytestmark = pytest.mark.gpu
@@ -109,16 +110,28 @@ def test_backward_in_groups(width, height, channels, tail):
 
 
 # Grids of 4096 to 6143 tiles: two pixels per lane beyond 40 list entries per
-# Gaussian, one up to them, and 8 channels in a further window after 56.
-@pytest.mark.parametrize("n,channels", [(400, 3), (17_000, 3), (400, 58), (17_000, 58)])
-def test_backward_of_mid_size_grids(n, channels):
+# Gaussian or where their count is not given, one up to 40, and 8 channels in a
+# further window after 56.
+@pytest.mark.parametrize("n,channels,counted", [(400, 3, True), (17_000, 3, True), (17_000, 3, False),
+                                                (400, 58, True), (17_000, 58, True)])
+def test_backward_of_mid_size_grids(n, channels, counted, monkeypatch):
     width, height = 1152, 960
-    print("backward mid-size grid", n, channels, flush=True)
+    print("backward mid-size grid", n, channels, counted, flush=True)
+    if not counted:
+        real, calls = native.call, []
+
+        def call(name, *args):
+            if name == "gs3d_render_bwd_lists":
+                calls.append(name)
+                return real("gs3d_render_bwd", args[0], args[2])
+            return real(name, *args)
+        monkeypatch.setattr(native, "call", call)
     centers, conics, feats, g = _scene(width, height, n, channels, extreme=False)
     ids, ranges = _lists(n, width, height, 150, g)
     assert 4096 <= len(ranges) < 6144 and (ids.numel() > 40 * n) == (n == 400)
     up = torch.randn((1, height, width, channels + 1), generator=g).to(DEV)
     got, ref, bound = _backward(width, height, ranges, ids, centers, conics, feats, up)
+    assert counted or len(calls) == 1
     for name in got:
         check_gradient(name, got[name], ref[name], bound[name])
 
